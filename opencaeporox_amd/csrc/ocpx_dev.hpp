@@ -48,6 +48,21 @@ struct DevSat {
     double sgof[4 * OCPX_MAX_TABROWS];
 };
 
+// Work items (cells, trials or teams) a persistent wavefront holds at once: a
+// queue shorter than the launch's lanes is dealt evenly over its wavefronts
+// instead of 64 to each of the first few.  A wavefront runs the union of its
+// lanes' branches and ends with its slowest lane, and an FP64 instruction
+// costs the same for one lane as for 64, so on an idle device fewer items per
+// wavefront only shorten the launch; a queue of at least (wavefronts * per)
+// items fills every lane as before.  Items are independent, so results do not
+// depend on it.
+__device__ __forceinline__ int items_per_wave(unsigned total, int per)
+{
+    const unsigned w = gridDim.x;                // 64-lane blocks
+    const unsigned l = (total + w - 1) / w;
+    return l < 1u ? 1 : (l > (unsigned)per ? per : (int)l);
+}
+
 // finite test usable on host and device (v - v is NaN for inf and NaN)
 OCPX_HD bool finite_d(double v) { return (v - v) == 0.0; }
 

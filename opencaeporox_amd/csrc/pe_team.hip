@@ -1005,12 +1005,22 @@ __global__ void __launch_bounds__(64) pe_team_batched(const DevFluid* __restrict
     const int lane = __lane_id();
     const int lead = lane & ~(T - 1);
     constexpr int NR_BATCH = (64 / T) / 4;
+    const unsigned nq = io.nq ? *io.nq : (unsigned)io.nb;
+    if (nq == 0) return;
+    // teams of 16 spread a short queue over the wavefronts: the restart loops
+    // of a flash's last cells then have a wavefront each (12,000 to 20,000
+    // cells: 5.45 -> 2.79 ms at Nc = 11, 3.79 -> 2.61 at Nc = 9, 7.56 -> 4.84
+    // at Nc = 12).  Smaller teams fill a wavefront as before: the loops of
+    // more wavefronts on a compute unit than fit its instruction cache cost
+    // them more than their neighbours' branches do (Nc = 6, T = 8, 1,000
+    // cells: 442 -> 462 us; a pass of a 10x10x10 grid 3.03 -> 3.49 ms).
+    const int tpw = T == 16 ? items_per_wave(nq, 64 / T) : 64 / T;
+    const int nr_batch = tpw / 4 > 1 ? tpw / 4 : 1;
     LaneFluid<NC, T> lf;
     Cell<NC, T> C;
     C.st = ST_DONE;
     C.model = 0;
-    bool have = false, drained = false;
-    const unsigned nq = io.nq ? *io.nq : (unsigned)io.nb;
+    bool have = false, drained = lane / T >= tpw;
     while (true) {
         if (C.st == ST_DONE && have) { end<NC, T>(io, C, ln); have = false; }
         const bool need = !have && !drained;
@@ -1040,7 +1050,7 @@ __global__ void __launch_bounds__(64) pe_team_batched(const DevFluid* __restrict
         if constexpr (NR_BATCH > 1) {
             const bool nr = live && (C.st == ST_T_NR || C.st == ST_S_NR);
             const unsigned long long mnr = __ballot(nr && ln.t == 0), mlive = __ballot(live && ln.t == 0);
-            const bool run_nr = __popcll(mnr) >= NR_BATCH || mnr == mlive;
+            const bool run_nr = __popcll(mnr) >= nr_batch || mnr == mlive;
             if (live && (!nr || run_nr)) step<NC, T>(fluid_of<NC, T, MULTI>(fp, C), lf, io, C, ln);
         } else if (live) {
             step<NC, T>(fluid_of<NC, T, MULTI>(fp, C), lf, io, C, ln);
@@ -1059,7 +1069,8 @@ hipError_t launch(const DevFluid* f, const PeIO& io, bool batched, int grid_bloc
         if (multi) return hipErrorInvalidValue;
         hipLaunchKernelGGL((pe_team_plain<NC, T, false>), dim3((unsigned)need), dim3(64), 0, st, f, io);
     } else {
-        const long nblk = grid_blocks < need ? grid_blocks : need;
+        const long most = T == 16 ? io.nb : need;    // teams of 16 spread a short queue over the grid
+        const long nblk = grid_blocks < most ? grid_blocks : most;
         if (multi) hipLaunchKernelGGL((pe_team_batched<NC, T, true>), dim3((unsigned)nblk), dim3(64), 0, st, f, io);
         else hipLaunchKernelGGL((pe_team_batched<NC, T, false>), dim3((unsigned)nblk), dim3(64), 0, st, f, io);
     }
