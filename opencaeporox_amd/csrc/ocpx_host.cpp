@@ -162,9 +162,13 @@ int dalloc(ocpx_ctx* c, T** p, size_t count)
     void* q = nullptr;
     hipError_t e = hipMalloc(&q, count * sizeof(T));
     if (e != hipSuccess) return fail(c, OCPX_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
-    e = hipMemset(q, 0, count * sizeof(T));
-    if (e != hipSuccess) return fail(c, OCPX_E_HIP, std::string("hipMemset: ") + hipGetErrorString(e));
     c->allocs.push_back(q);
+    // zeroed on the context's stream and waited for: a caller's stream need not
+    // be ordered with the default one (torch's are not), so a fill there could
+    // run after the context's next kernels or copies
+    e = hipMemsetAsync(q, 0, count * sizeof(T), c->st);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->st);
+    if (e != hipSuccess) return fail(c, OCPX_E_HIP, std::string("hipMemset: ") + hipGetErrorString(e));
     *p = (T*)q;
     return OCPX_OK;
 }
