@@ -128,6 +128,45 @@ inline bool coarsen(const Graph& g, Graph& gc, LevelMaps& L)
     return true;
 }
 
+// One level's matrix in the order the V-cycle's kernels walk it: position
+// q = 4 I + m is the m-th member row of aggregate I (row[q], -1 when the
+// aggregate has fewer), 64 positions to a slice, and entry k of the slice's
+// lane at off[slice] + 64 k + lane, so a wavefront's loads are contiguous and
+// an aggregate's four rows sit in neighbouring lanes.  src is the entry's CSR
+// slot (-1: padding, whose column is a valid row and whose value stays 0);
+// cagg the aggregate of its column.
+struct Sell {
+    std::vector<int64_t> off;
+    std::vector<int32_t> row, ci, cagg, src;
+};
+
+inline void sell_layout(const Graph& g, const LevelMaps& L, int64_t nc, Sell& s)
+{
+    const int64_t nq = (4 * nc + 63) / 64 * 64;
+    s.row.assign(nq, -1);
+    for (int64_t I = 0; I < nc; I++)
+        for (int64_t k = L.mp[I]; k < L.mp[I + 1]; k++) s.row[4 * I + (k - L.mp[I])] = L.mi[k];
+    s.off.assign(1, 0);
+    s.ci.clear();
+    s.cagg.clear();
+    s.src.clear();
+    for (int64_t q0 = 0; q0 < nq; q0 += 64) {
+        int64_t w = 0;
+        for (int64_t q = q0; q < q0 + 64; q++)
+            if (s.row[q] >= 0) w = std::max(w, g.rp[s.row[q] + 1] - g.rp[s.row[q]]);
+        for (int64_t k = 0; k < w; k++)
+            for (int64_t q = q0; q < q0 + 64; q++) {
+                const int64_t i = s.row[q];
+                const bool in = i >= 0 && g.rp[i] + k < g.rp[i + 1];
+                const int32_t c = in ? g.ci[g.rp[i] + k] : (int32_t)(i >= 0 ? i : 0);
+                s.ci.push_back(c);
+                s.cagg.push_back(L.agg[c]);
+                s.src.push_back(in ? (int32_t)(g.rp[i] + k) : -1);
+            }
+        s.off.push_back((int64_t)s.ci.size());
+    }
+}
+
 // Greedy colouring of a block graph (rowptr, col) in row order: colour
 // lists rows[cptr[c] .. cptr[c+1]) in ascending row order; no two rows of one
 // colour are neighbours.

@@ -3,9 +3,10 @@
 // cpr.hpp).
 //
 // Every kernel here is a plain gather: a thread (or a group of B lanes for a
-// block row) owns its output entries, so no atomics and the same bits on
-// every run.  The AMG level matrices are scalar CSR with the diagonal first
-// in each row.
+// block row) owns its output entries and reductions sum in a fixed order, so
+// the same bits on every run.  The AMG level matrices are formed as scalar CSR
+// with the diagonal first in each row and walked by the V-cycle in sliced
+// columns (amg::Sell).
 #include <algorithm>
 #include <cstring>
 
@@ -17,41 +18,58 @@ namespace ocpx {
 
 namespace {
 
-constexpr double OMEGA = 2.0 / 3.0;          // weighted-Jacobi smoother
+constexpr double OMEGA = PressureAmg::OMEGA;
 constexpr int MAX_LEVELS = 25;
 
 // ------------------------------------------------------------------ kernels
-// level 0: a[s] = sum_m Dinv_i(0, m) A_s(m, 0), one thread per block row i,
-// made an M-matrix for the hierarchy: positive off-diagonal entries go to
-// the diagonal, and the diagonal is at least the sum of the remaining
-// off-diagonal magnitudes (the decoupled pressure block of a state far from
-// equilibrium is indefinite, and a Jacobi-smoothed aggregation cycle on it
-// diverges)
-__global__ void __launch_bounds__(256) amg_l0(int B, int64_t n, const int64_t* __restrict__ rp,
-                                              const double* __restrict__ val, const double* __restrict__ dinv,
-                                              double* __restrict__ a)
+// Column 0 of every decoupled block, d0[s] = Dinv_i A_s(:, 0), by B lanes per
+// block row (lane r = row r; the block's column is passed round the lanes),
+// and from its row 0 the pressure block a[s], made an M-matrix for the
+// hierarchy: positive off-diagonal entries go to the diagonal, and the
+// diagonal is at least the sum of the remaining off-diagonal magnitudes (the
+// decoupled pressure block of a state far from equilibrium is indefinite, and a
+// Jacobi-smoothed aggregation cycle on it diverges).  The correction of the
+// pressure stage is non-zero in the pressures only, so its residual needs
+// these columns and not the blocks: 1 / B of the matrix.
+template <int B>
+__global__ void __launch_bounds__(64) cpr_columns(int64_t n, const int64_t* __restrict__ rp,
+                                                  const double* __restrict__ val, const double* __restrict__ dinv,
+                                                  double* __restrict__ d0, double* __restrict__ a)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const double* d = dinv + (size_t)i * B * B;     // row 0 of Dinv_i
-    const size_t BB = (size_t)B * B;
-    const int64_t s0 = rp[i], s1 = rp[i + 1];       // the diagonal slot first
+    constexpr int G = 64 / B;
+    const int lane = threadIdx.x, g = lane / B, r = lane % B;
+    const int64_t i = (int64_t)blockIdx.x * G + g;
+    const bool valid = g < G && i < n;
+    const int base = (g < G ? g : 0) * B;
+    double d[B];
+    UNROLL for (int m = 0; m < B; m++) d[m] = valid ? dinv[((size_t)i * B + r) * B + m] : 0.0;
+    const int64_t s0 = valid ? rp[i] : 0, s1 = valid ? rp[i + 1] : 0;
+    int cnt = (int)(s1 - s0);                       // the wavefront runs its longest row, so every
+    for (int o = 32; o > 0; o >>= 1) cnt = max(cnt, __shfl_xor(cnt, o));   // lane takes part in the exchanges
     double diag = 0, pos = 0, neg = 0;
-    for (int64_t s = s0; s < s1; s++) {
-        const double* blk = val + (size_t)s * BB;
+    for (int k = 0; k < cnt; k++) {
+        const int64_t s = s0 + k;
+        const bool in = s < s1;
+        const double c = in ? val[((size_t)s * B + r) * B] : 0.0;
         double acc = 0;
-        for (int m = 0; m < B; m++) acc += d[m] * blk[(size_t)m * B];
-        if (s == s0) {
-            diag = acc;
-        } else if (acc > 0) {
-            pos += acc;
-            acc = 0;
-        } else {
-            neg -= acc;
+        UNROLL for (int m = 0; m < B; m++) acc += d[m] * __shfl(c, base + m);
+        if (!in) continue;
+        d0[(size_t)s * B + r] = acc;
+        if (r == 0) {
+            if (k == 0) {
+                diag = acc;
+            } else {
+                if (acc > 0) {
+                    pos += acc;
+                    acc = 0;
+                } else {
+                    neg -= acc;
+                }
+                a[s] = acc;
+            }
         }
-        a[s] = acc;
     }
-    a[s0] = fmax(diag + pos, neg);
+    if (valid && r == 0) a[s0] = fmax(diag + pos, neg);
 }
 
 __global__ void __launch_bounds__(256) amg_gather(int64_t nnz, const int64_t* __restrict__ gp,
@@ -74,13 +92,14 @@ __global__ void __launch_bounds__(256) amg_dinv(int64_t n, const int64_t* __rest
     dinv[i] = d != 0 ? 1 / d : 0.0;
 }
 
-// x = OMEGA Dinv b (a sweep from x = 0)
-__global__ void __launch_bounds__(256) amg_smooth0(int64_t n, const double* __restrict__ dinv,
-                                                   const double* __restrict__ b, double* __restrict__ x)
+// a level's values in V-cycle order
+__global__ void __launch_bounds__(256) amg_sell(int64_t ne, const int32_t* __restrict__ src,
+                                                const double* __restrict__ a, double* __restrict__ sa)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    x[i] = OMEGA * dinv[i] * b[i];
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= ne) return;
+    const int32_t s = src[e];
+    sa[e] = s >= 0 ? a[s] : 0.0;
 }
 
 // xo = x + OMEGA Dinv (b - A x)
@@ -96,33 +115,138 @@ __global__ void __launch_bounds__(256) amg_smooth(int64_t n, const int64_t* __re
     xo[i] = x[i] + OMEGA * dinv[i] * r;
 }
 
-// bc[I] = sum over the rows i of aggregate I of (b - A x)[i]
-__global__ void __launch_bounds__(256) amg_resid_restrict(int64_t nc, const int64_t* __restrict__ mp,
-                                                          const int32_t* __restrict__ mi,
-                                                          const int64_t* __restrict__ rp,
-                                                          const int32_t* __restrict__ ci,
-                                                          const double* __restrict__ a,
-                                                          const double* __restrict__ b,
-                                                          const double* __restrict__ x, double* __restrict__ bc)
+// Down a level: the residual of each position's row, summed over the
+// aggregate's four positions, is the coarse right-hand side; the coarse level's
+// first sweep from zero, OMEGA Dinv b, is written with it.  The thread per
+// fine row (a thread per coarse row walked its rows one after another: 72 us at
+// 500,000 rows, 22 now) and the sliced columns keep every load of the matrix
+// contiguous.
+__global__ void __launch_bounds__(256) amg_down(int64_t nq, int64_t nc, const int64_t* __restrict__ off,
+                                                const int32_t* __restrict__ row, const int32_t* __restrict__ ci,
+                                                const double* __restrict__ a, const double* __restrict__ b,
+                                                const double* __restrict__ x, const double* __restrict__ dinvc,
+                                                double* __restrict__ bc, double* __restrict__ xc)
 {
-    const int64_t I = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (I >= nc) return;
-    double acc = 0;
-    for (int64_t k = mp[I]; k < mp[I + 1]; k++) {
-        const int64_t i = mi[k];
-        double r = b[i];
-        for (int64_t s = rp[i]; s < rp[i + 1]; s++) r -= a[s] * x[ci[s]];
-        acc += r;
+    const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (q >= nq) return;                            // nq is a multiple of 64: whole wavefronts
+    const int32_t i = row[q];
+    double r = 0;
+    if (i >= 0) {
+        r = b[i];
+        const int64_t e1 = off[(q >> 6) + 1];
+        for (int64_t e = off[q >> 6] + (q & 63); e < e1; e += 64) r -= a[e] * x[ci[e]];
     }
-    bc[I] = acc;
+    r += __shfl_xor(r, 1);
+    r += __shfl_xor(r, 2);
+    const int64_t I = q >> 2;
+    if ((q & 3) == 0 && I < nc) {
+        bc[I] = r;
+        xc[I] = OMEGA * dinvc[I] * r;
+    }
 }
 
-__global__ void __launch_bounds__(256) amg_prolong(int64_t n, const int32_t* __restrict__ agg,
-                                                   const double* __restrict__ xc, double* __restrict__ x)
+// Up a level: x' = x + the coarse correction of the row's aggregate, then one
+// weighted-Jacobi sweep, both in one pass (cagg: the aggregate of a column).
+__global__ void __launch_bounds__(256) amg_up(int64_t nq, const int64_t* __restrict__ off,
+                                              const int32_t* __restrict__ row, const int32_t* __restrict__ ci,
+                                              const int32_t* __restrict__ cagg, const double* __restrict__ a,
+                                              const double* __restrict__ dinv, const double* __restrict__ b,
+                                              const double* __restrict__ x, const double* __restrict__ xc,
+                                              double* __restrict__ xo)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    x[i] += xc[agg[i]];
+    const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (q >= nq) return;
+    const int32_t i = row[q];
+    if (i < 0) return;
+    double r = b[i];
+    const int64_t e1 = off[(q >> 6) + 1];
+    for (int64_t e = off[q >> 6] + (q & 63); e < e1; e += 64) r -= a[e] * (x[ci[e]] + xc[cagg[e]]);
+    xo[i] = (x[i] + xc[q >> 2]) + OMEGA * dinv[i] * r;
+}
+
+// The part of the V-cycle below about 2,000 rows in one workgroup: every
+// vector in LDS, the matrices read from L2, the coarsest level by its dense
+// inverse.  Launched level by level, those levels took four launches each and
+// a serial triangular solve (27 us), about 150 us of the cycle's 550 at
+// 500,000 rows; this kernel takes 25.
+constexpr int SM_ROWS = 3072, SM_TOP = 2048, SM_LEVELS = 14, SM_THREADS = 1024;
+struct SmallLevel {
+    int n, nc, nq;
+    const int64_t* off;
+    const int32_t *row, *ci, *cagg;
+    const double *a, *dinv;
+};
+struct SmallHier {
+    int nl, nd;                              // levels above the dense one, rows of the dense one
+    const double *inv, *dinvd;
+    SmallLevel lv[SM_LEVELS];
+};
+
+__global__ void __launch_bounds__(SM_THREADS) amg_small(SmallHier h, const double* __restrict__ b,
+                                                        double* __restrict__ xo)
+{
+    constexpr int N = PressureAmg::DENSE_MAX;
+    __shared__ double sb[SM_ROWS], sx[SM_ROWS], so[SM_TOP];
+    const int t = threadIdx.x;
+    const int n0 = h.nl ? h.lv[0].n : h.nd;
+    const double* d0 = h.nl ? h.lv[0].dinv : h.dinvd;
+    for (int i = t; i < n0; i += SM_THREADS) {
+        const double v = b[i];
+        sb[i] = v;
+        sx[i] = OMEGA * d0[i] * v;
+    }
+    __syncthreads();
+    int o = 0;
+    for (int l = 0; l < h.nl; l++) {
+        const SmallLevel& L = h.lv[l];
+        const int on = o + L.n;
+        const double* dn = l + 1 < h.nl ? h.lv[l + 1].dinv : h.dinvd;
+        for (int q = t; q < L.nq; q += SM_THREADS) {         // nq is a multiple of 64: whole wavefronts
+            const int i = L.row[q];
+            double r = 0;
+            if (i >= 0) {
+                r = sb[o + i];
+                const int e1 = (int)L.off[(q >> 6) + 1];
+                for (int e = (int)L.off[q >> 6] + (q & 63); e < e1; e += 64) r -= L.a[e] * sx[o + L.ci[e]];
+            }
+            r += __shfl_xor(r, 1);
+            r += __shfl_xor(r, 2);
+            const int I = q >> 2;
+            if ((q & 3) == 0 && I < L.nc) {
+                sb[on + I] = r;
+                sx[on + I] = OMEGA * dn[I] * r;
+            }
+        }
+        __syncthreads();
+        o = on;
+    }
+    {   // sixteen lanes per row of the dense inverse
+        const int i = t >> 4, c = t & 15;
+        double acc = 0;
+        if (i < h.nd)
+            for (int j = c; j < h.nd; j += 16) acc += h.inv[i * N + j] * sb[o + j];
+        for (int m = 8; m > 0; m >>= 1) acc += __shfl_xor(acc, m);
+        if (i < h.nd && c == 0) sx[o + i] = acc;
+    }
+    __syncthreads();
+    for (int l = h.nl - 1; l >= 0; l--) {
+        const SmallLevel& L = h.lv[l];
+        const int on = o;
+        o -= L.n;
+        for (int q = t; q < L.nq; q += SM_THREADS) {
+            const int i = L.row[q];
+            if (i < 0) continue;
+            double r = sb[o + i];
+            const int e1 = (int)L.off[(q >> 6) + 1];
+            for (int e = (int)L.off[q >> 6] + (q & 63); e < e1; e += 64)
+                r -= L.a[e] * (sx[o + L.ci[e]] + sx[on + L.cagg[e]]);
+            so[i] = (sx[o + i] + sx[on + (q >> 2)]) + OMEGA * L.dinv[i] * r;
+        }
+        __syncthreads();
+        for (int i = t; i < L.n; i += SM_THREADS) sx[o + i] = so[i];
+        __syncthreads();
+    }
+    for (int i = t; i < n0; i += SM_THREADS) xo[i] = sx[i];
 }
 
 // Dense LU with partial pivoting of the coarsest level (n <= 64), one
@@ -167,32 +291,31 @@ __global__ void __launch_bounds__(64) amg_dense_lu(int n, const int64_t* __restr
     for (int j = 0; j < N; j++) lu[t * N + j] = M[t][j];
 }
 
-__global__ void __launch_bounds__(64) amg_dense_solve(int n, const double* __restrict__ lu,
-                                                      const int32_t* __restrict__ piv, const double* __restrict__ b,
-                                                      double* __restrict__ x)
+// The coarsest level's inverse from its LU, lane t = column t: once per solve,
+// so each cycle's coarsest solve is one product.
+__global__ void __launch_bounds__(64) amg_dense_inv(int n, const double* __restrict__ lu,
+                                                    const int32_t* __restrict__ piv, double* __restrict__ inv)
 {
     constexpr int N = PressureAmg::DENSE_MAX;
-    __shared__ double y[N];
+    __shared__ double M[N * N], Y[N * N];
     const int t = threadIdx.x;
-    y[t] = t < n ? b[t] : 0.0;
+    for (int i = 0; i < N; i++) { M[i * N + t] = lu[i * N + t]; Y[i * N + t] = i == t ? 1.0 : 0.0; }
     __syncthreads();
-    if (t == 0)
-        for (int k = 0; k < n; k++) {
-            const int p = piv[k];
-            if (p != k) { const double v = y[k]; y[k] = y[p]; y[p] = v; }
-        }
-    __syncthreads();
-    for (int k = 0; k < n; k++) {        // L (unit diagonal)
-        if (t > k && t < n) y[t] -= lu[t * N + k] * y[k];
-        __syncthreads();
+    for (int k = 0; k < n; k++) {
+        const int p = piv[k];
+        if (p != k) { const double v = Y[k * N + t]; Y[k * N + t] = Y[p * N + t]; Y[p * N + t] = v; }
     }
-    for (int k = n - 1; k >= 0; k--) {   // U
-        if (t == k) y[k] = lu[k * N + k] != 0 ? y[k] / lu[k * N + k] : 0.0;
-        __syncthreads();
-        if (t < k) y[t] -= lu[t * N + k] * y[k];
-        __syncthreads();
+    for (int i = 0; i < n; i++) {        // L (unit diagonal); a lane reads and writes its own column only
+        double v = Y[i * N + t];
+        for (int k = 0; k < i; k++) v -= M[i * N + k] * Y[k * N + t];
+        Y[i * N + t] = v;
     }
-    if (t < n) x[t] = y[t];
+    for (int i = n - 1; i >= 0; i--) {   // U
+        double v = Y[i * N + t];
+        for (int k = i + 1; k < n; k++) v -= M[i * N + k] * Y[k * N + t];
+        Y[i * N + t] = M[i * N + i] != 0 ? v / M[i * N + i] : 0.0;
+    }
+    for (int i = 0; i < N; i++) inv[i * N + t] = (i < n && t < n) ? Y[i * N + t] : 0.0;
 }
 
 // One colour of the block Gauss-Seidel sweep; a group of B lanes per row,
@@ -225,76 +348,212 @@ __global__ void __launch_bounds__(64) gs_color(const int32_t* __restrict__ rows,
     if (valid) x[(size_t)i * B + r] = y;
 }
 
-constexpr int MD_BLOCKS = 512, MD_THREADS = 256, MD_MAX = 32;
-
-// part[k][blockIdx.x] = partial sums of V_k . w over a fixed slice
-__global__ void __launch_bounds__(MD_THREADS) mdot_part(const double* __restrict__ V, int64_t ldv, int m,
-                                                        const double* __restrict__ w, int64_t len,
-                                                        double* __restrict__ part)
+// R = v - Dinv J x1 and z = R + x1 on the bulk rows for the pressure
+// correction x1 (px in the pressure entries, 0 elsewhere).
+template <int B>
+__global__ void __launch_bounds__(64) cpr_resid(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ col,
+                                                const double* __restrict__ d0, const double* __restrict__ px,
+                                                const double* __restrict__ v, double* __restrict__ R,
+                                                double* __restrict__ z, int64_t nb)
 {
-    __shared__ double sh[MD_THREADS];
-    const int t = threadIdx.x;
-    for (int k = 0; k < m; k++) {
-        const double* v = V + (size_t)k * ldv;
-        double acc = 0;
-        for (int64_t i = (int64_t)blockIdx.x * MD_THREADS + t; i < len; i += (int64_t)MD_BLOCKS * MD_THREADS)
-            acc += v[i] * w[i];
-        sh[t] = acc;
-        __syncthreads();
-        for (int s = MD_THREADS / 2; s > 0; s >>= 1) {
-            if (t < s) sh[t] += sh[t + s];
-            __syncthreads();
+    constexpr int G = 64 / B;
+    const int lane = threadIdx.x, g = lane / B, r = lane % B;
+    const int64_t i = (int64_t)blockIdx.x * G + g;
+    if (g >= G || i >= nb) return;
+    double t = 0;
+    for (int64_t s = rowptr[i]; s < rowptr[i + 1]; s++) t += d0[(size_t)s * B + r] * px[col[s]];
+    const double y = v[(size_t)i * B + r] - t;
+    R[(size_t)i * B + r] = y;
+    z[(size_t)i * B + r] = r == 0 ? y + px[i] : y;
+}
+
+// The Gauss-Seidel sweep and the operator after it on a two-coloured graph,
+// with the matrix read once.  g = the sweep from zero on D^{-1} J g = R: the
+// first colour's rows keep R (their neighbours are still zero), the second
+// colour's are g2 = R2 - Dinv A21 R1 (SECOND), z = g + x1.  Then w = D^{-1} J z =
+// D^{-1} J g + (v - R); the sweep solved the second colour's rows exactly, so w2 =
+// v2, and w1 = R1 + Dinv A12 g2 + v1 - R1 = v1 + Dinv A12 g2 (first colour).
+// R holds g afterwards.  One iteration reads the off-diagonal blocks once; the
+// sweep over both colours, the residual before it and the product after it read
+// the matrix three times (500,000 rows, B = 8: 0.47 + 0.36 + 0.36 ms, now 0.45).
+template <int B, bool SECOND>
+__global__ void __launch_bounds__(64) cpr_half(const int32_t* __restrict__ rows, int64_t nrows,
+                                               const int64_t* __restrict__ rowptr, const int32_t* __restrict__ col,
+                                               const double* __restrict__ val, const double* __restrict__ dinv,
+                                               const double* __restrict__ px, const double* __restrict__ v,
+                                               double* R, double* __restrict__ z, double* __restrict__ w)
+{
+    constexpr int G = 64 / B;
+    const int lane = threadIdx.x, g = lane / B, r = lane % B;
+    const int64_t k = (int64_t)blockIdx.x * G + g;
+    const bool valid = g < G && k < nrows;
+    const int64_t i = valid ? rows[k] : 0;
+    double t = 0;
+    if (valid)
+        for (int64_t s = rowptr[i] + 1; s < rowptr[i + 1]; s++) {
+            const double* blk = val + ((size_t)s * B + r) * B;
+            const double* xm = R + (size_t)col[s] * B;
+            UNROLL for (int c = 0; c < B; c++) t += blk[c] * xm[c];
         }
-        if (t == 0) part[(size_t)k * MD_BLOCKS + blockIdx.x] = sh[0];
-        __syncthreads();
+    const int base = (g < G ? g : 0) * B;
+    const double* d = dinv + ((size_t)i * B + r) * B;
+    double y = 0;
+    UNROLL for (int c = 0; c < B; c++) {
+        const double tc = __shfl(t, base + c);
+        if (valid) y += d[c] * tc;
+    }
+    if (!valid) return;
+    const size_t o = (size_t)i * B + r;
+    if constexpr (SECOND) {
+        const double gi = R[o] - y;
+        R[o] = gi;
+        z[o] = r == 0 ? gi + px[i] : gi;
+        w[o] = v[o];
+    } else {
+        w[o] = v[o] + y;
     }
 }
 
-__global__ void __launch_bounds__(MD_THREADS) mdot_final(int m, const double* __restrict__ part,
-                                                         double* __restrict__ out)
-{
-    __shared__ double sh[MD_THREADS];
-    const int t = threadIdx.x;
-    for (int k = 0; k < m; k++) {
-        double acc = 0;
-        for (int j = t; j < MD_BLOCKS; j += MD_THREADS) acc += part[(size_t)k * MD_BLOCKS + j];
-        sh[t] = acc;
-        __syncthreads();
-        for (int s = MD_THREADS / 2; s > 0; s >>= 1) {
-            if (t < s) sh[t] += sh[t + s];
-            __syncthreads();
-        }
-        if (t == 0) out[k] = sh[0];
-        __syncthreads();
-    }
-}
+// ------------------------------------------------- Gram-Schmidt of one vector
+// Classical Gram-Schmidt with one reorthogonalisation against M vectors in
+// three passes over them (h = V.w; w -= V h with h2 = V.w; w -= V h2 with w.w),
+// each element's M values held in registers, the partials summed by the last
+// block to finish.  Bandwidth-bound: a pass reads M + 1 vectors.  One pass per
+// product and per update, each reading w again for every vector, took 26 ms of
+// a 45-iteration solve of 4M unknowns; these take 14.
+constexpr int FG_THREADS = 256, FG_BLOCKS = 512, FG_MAX = 31;
 
-__global__ void __launch_bounds__(256) maxpy(double* __restrict__ w, const double* __restrict__ V, int64_t ldv,
-                                             int m, const double* __restrict__ h, int64_t len)
+// sums acc over the block into part, and returns true in the last block of
+// the grid, which then finds the M totals in tot (LDS, valid after the call)
+template <int M>
+__device__ __forceinline__ bool fg_reduce(double (&acc)[M], double* part, unsigned* done, double* tot)
 {
-    __shared__ double hs[MD_MAX];
-    if (threadIdx.x < m) hs[threadIdx.x] = h[threadIdx.x];
+    __shared__ double sh[FG_THREADS / 64][32];
+    __shared__ double sums[8][32];
+    __shared__ bool last;
+    const int t = threadIdx.x, wv = t >> 6, ln = t & 63;
+    UNROLL for (int k = 0; k < M; k++) {
+        double v = acc[k];
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+        if (ln == 0) sh[wv][k] = v;
+    }
     __syncthreads();
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= len) return;
-    double acc = w[i];
-    for (int k = 0; k < m; k++) acc += hs[k] * V[(size_t)k * ldv + i];
-    w[i] = acc;
+    if (t < M) part[(size_t)blockIdx.x * 32 + t] = ((sh[0][t] + sh[1][t]) + sh[2][t]) + sh[3][t];
+    __threadfence();
+    __syncthreads();
+    if (t == 0) last = atomicAdd(done, 1u) == gridDim.x - 1;
+    __syncthreads();
+    if (!last) return false;
+    __threadfence();
+    const int k = t & 31, g = t >> 5;
+    double v = 0;
+    if (k < M)
+        for (unsigned b = g; b < gridDim.x; b += 8) v += __builtin_nontemporal_load(&part[(size_t)b * 32 + k]);
+    sums[g][k] = v;
+    __syncthreads();
+    if (t < M) {
+        double u = 0;
+        for (int q = 0; q < 8; q++) u += sums[q][t];
+        tot[t] = u;
+    }
+    if (t == 0) *done = 0;
+    __syncthreads();
+    return true;
 }
 
-__global__ void __launch_bounds__(256) gather_p(int B, const double* __restrict__ v, double* __restrict__ p, int64_t n)
+template <int M>
+__global__ void __launch_bounds__(FG_THREADS) fg_dot(const double* __restrict__ V, int64_t ldv,
+                                                     const double* __restrict__ w, int64_t len, double* part,
+                                                     unsigned* done, double* __restrict__ h, double* host)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) p[i] = v[(size_t)i * B];
+    __shared__ double tot[32];
+    double acc[M];
+    UNROLL for (int k = 0; k < M; k++) acc[k] = 0;
+    for (int64_t i = (int64_t)blockIdx.x * FG_THREADS + threadIdx.x; i < len; i += (int64_t)gridDim.x * FG_THREADS) {
+        const double wi = w[i];
+        UNROLL for (int k = 0; k < M; k++) acc[k] += V[(size_t)k * ldv + i] * wi;
+    }
+    if (!fg_reduce<M>(acc, part, done, tot)) return;
+    if (threadIdx.x < M) {
+        h[threadIdx.x] = tot[threadIdx.x];
+        if (host) host[threadIdx.x] = tot[threadIdx.x];
+    }
 }
 
-__global__ void __launch_bounds__(256) scatter_p(int B, const double* __restrict__ p, double* __restrict__ v,
-                                                 int64_t n, int64_t len)
+template <int M>
+__global__ void __launch_bounds__(FG_THREADS) fg_orth(double* __restrict__ w, const double* __restrict__ V,
+                                                      int64_t ldv, const double* __restrict__ h, int64_t len,
+                                                      double* part, unsigned* done, double* __restrict__ h2)
+{
+    __shared__ double tot[32], hs[32];
+    if (threadIdx.x < M) hs[threadIdx.x] = h[threadIdx.x];
+    __syncthreads();
+    double acc[M];
+    UNROLL for (int k = 0; k < M; k++) acc[k] = 0;
+    for (int64_t i = (int64_t)blockIdx.x * FG_THREADS + threadIdx.x; i < len; i += (int64_t)gridDim.x * FG_THREADS) {
+        double v[M];
+        UNROLL for (int k = 0; k < M; k++) v[k] = V[(size_t)k * ldv + i];
+        double wi = w[i];
+        UNROLL for (int k = 0; k < M; k++) wi -= hs[k] * v[k];
+        w[i] = wi;
+        UNROLL for (int k = 0; k < M; k++) acc[k] += v[k] * wi;
+    }
+    if (!fg_reduce<M>(acc, part, done, tot)) return;
+    if (threadIdx.x < M) h2[threadIdx.x] = tot[threadIdx.x];
+}
+
+template <int M>
+__global__ void __launch_bounds__(FG_THREADS) fg_orth_norm(double* __restrict__ w, const double* __restrict__ V,
+                                                           int64_t ldv, const double* __restrict__ h,
+                                                           const double* __restrict__ h2, int64_t len, double* part,
+                                                           unsigned* done, double* host, double* __restrict__ scale)
+{
+    __shared__ double tot[32], hs[32];
+    const int t = threadIdx.x;
+    if (t < M) hs[t] = h2[t];
+    __syncthreads();
+    double acc[1] = {0};
+    for (int64_t i = (int64_t)blockIdx.x * FG_THREADS + t; i < len; i += (int64_t)gridDim.x * FG_THREADS) {
+        double v[M];
+        UNROLL for (int k = 0; k < M; k++) v[k] = V[(size_t)k * ldv + i];
+        double wi = w[i];
+        UNROLL for (int k = 0; k < M; k++) wi -= hs[k] * v[k];
+        w[i] = wi;
+        acc[0] += wi * wi;
+    }
+    if (!fg_reduce<1>(acc, part, done, tot)) return;
+    if (t < M) host[t] = h[t] + hs[t];
+    if (t == 0) {
+        host[M] = tot[0];
+        *scale = 1 / sqrt(tot[0]);
+    }
+}
+
+template <int B>
+__global__ void __launch_bounds__(256) fg_scale(double* __restrict__ v, const double* __restrict__ w,
+                                                const double* __restrict__ scale, double s, int64_t nb, int64_t len,
+                                                const double* __restrict__ dinv0, double* __restrict__ pb,
+                                                double* __restrict__ px0)
 {
     const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (k >= len) return;
+    const double y = w[k] * (scale ? *scale : s);
+    v[k] = y;
     const int64_t i = k / B;
-    v[k] = (i < n && k == i * B) ? p[i] : 0.0;
+    if (k == i * B && i < nb) {
+        pb[i] = y;
+        px0[i] = OMEGA * dinv0[i] * y;
+    }
+}
+
+__global__ void __launch_bounds__(256) fg_axpy(double* __restrict__ x, const double* __restrict__ Z, int64_t ldz,
+                                               int m, FgCoef y, int64_t len)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= len) return;
+    double acc = x[i];
+    for (int k = 0; k < m; k++) acc += y.y[k] * Z[(size_t)k * ldz + i];
+    x[i] = acc;
 }
 
 unsigned grid256(int64_t n) { return (unsigned)((n + 255) / 256); }
@@ -347,80 +606,111 @@ int PressureAmg::setup(int64_t n, const std::vector<int64_t>& rp, const std::vec
             lv_.push_back(L);
             break;
         }
-        if (dev(&L.agg, M.agg.size(), M.agg.data(), err) || dev(&L.gp, M.gp.size(), M.gp.data(), err) ||
-            dev(&L.gs, M.gs.size(), M.gs.data(), err) || dev(&L.mp, M.mp.size(), M.mp.data(), err) ||
-            dev(&L.mi, M.mi.size(), M.mi.data(), err))
+        amg::Sell S;
+        amg::sell_layout(g, M, gc.n, S);
+        L.nc = gc.n;
+        L.nq = (int64_t)S.row.size();
+        L.ne = (int64_t)S.ci.size();
+        if (dev(&L.gp, M.gp.size(), M.gp.data(), err) || dev(&L.gs, M.gs.size(), M.gs.data(), err) ||
+            dev(&L.off, S.off.size(), S.off.data(), err) || dev(&L.row, S.row.size(), S.row.data(), err) ||
+            dev(&L.sci, S.ci.size(), S.ci.data(), err) || dev(&L.cagg, S.cagg.size(), S.cagg.data(), err) ||
+            dev(&L.src, S.src.size(), S.src.data(), err) || dev(&L.sa, (size_t)L.ne, (const double*)nullptr, err))
             return -1;
         lv_.push_back(L);
         g = std::move(gc);
     }
-    if (lv_.back().n <= DENSE_MAX &&
-        (dev(&lu_, (size_t)DENSE_MAX * DENSE_MAX, (const double*)nullptr, err) ||
-         dev(&piv_, (size_t)DENSE_MAX, (const int32_t*)nullptr, err)))
-        return -1;
-    rp0_ = lv_[0].rp;
+    if (lv_.back().n <= DENSE_MAX) {
+        if (dev(&lu_, (size_t)DENSE_MAX * DENSE_MAX, (const double*)nullptr, err) ||
+            dev(&inv_, (size_t)DENSE_MAX * DENSE_MAX, (const double*)nullptr, err) ||
+            dev(&piv_, (size_t)DENSE_MAX, (const int32_t*)nullptr, err))
+            return -1;
+        // the levels whose vectors fit one workgroup's LDS
+        int64_t rows = 0;
+        for (int l = (int)lv_.size() - 1; l >= 0; l--) {
+            rows += lv_[l].n;
+            if (lv_[l].n > SM_TOP || rows > SM_ROWS || (int)lv_.size() - 1 - l > SM_LEVELS) break;
+            small_ = l;
+        }
+    }
     return 0;
 }
 
-hipError_t PressureAmg::values(int B, const double* val, const double* dinv, hipStream_t st)
-{
-    Level& L0 = lv_[0];
-    hipLaunchKernelGGL(amg_l0, dim3(grid256(L0.n)), dim3(256), 0, st, B, L0.n, L0.rp, val, dinv, L0.a);
-    for (size_t l = 0; l < lv_.size(); l++) {
-        Level& L = lv_[l];
-        hipLaunchKernelGGL(amg_dinv, dim3(grid256(L.n)), dim3(256), 0, st, L.n, L.rp, L.a, L.dinv);
-        if (l + 1 < lv_.size()) {
-            Level& C = lv_[l + 1];
-            hipLaunchKernelGGL(amg_gather, dim3(grid256(C.nnz)), dim3(256), 0, st, C.nnz, L.gp, L.gs, L.a, C.a);
-        }
-    }
-    const Level& Lc = lv_.back();
-    if (Lc.n <= DENSE_MAX)
-        hipLaunchKernelGGL(amg_dense_lu, dim3(1), dim3(64), 0, st, (int)Lc.n, Lc.rp, Lc.ci, Lc.a, lu_, piv_);
-    return hipGetLastError();
-}
-
-hipError_t PressureAmg::cycle(int l, const double* b, double* x, hipStream_t st)
-{
-    Level& L = lv_[l];
-    if (l + 1 == (int)lv_.size()) {
-        if (L.n <= DENSE_MAX) {
-            hipLaunchKernelGGL(amg_dense_solve, dim3(1), dim3(64), 0, st, (int)L.n, lu_, piv_, b, x);
-        } else {                              // no dense level: a few sweeps
-            hipLaunchKernelGGL(amg_smooth0, dim3(grid256(L.n)), dim3(256), 0, st, L.n, L.dinv, b, L.r);
-            double *in = L.r, *out = x;
-            for (int k = 0; k < 9; k++) {
-                hipLaunchKernelGGL(amg_smooth, dim3(grid256(L.n)), dim3(256), 0, st, L.n, L.rp, L.ci, L.a, L.dinv,
-                                   b, in, out);
-                std::swap(in, out);
-            }
-            if (in != x) hipMemcpyAsync(x, in, (size_t)L.n * sizeof(double), hipMemcpyDeviceToDevice, st);
-        }
-        return hipGetLastError();
-    }
-    Level& C = lv_[l + 1];
-    hipLaunchKernelGGL(amg_smooth0, dim3(grid256(L.n)), dim3(256), 0, st, L.n, L.dinv, b, L.x);
-    hipLaunchKernelGGL(amg_resid_restrict, dim3(grid256(C.n)), dim3(256), 0, st, C.n, L.mp, L.mi, L.rp, L.ci, L.a,
-                       b, L.x, C.b);
-    hipError_t e = cycle(l + 1, C.b, C.x, st);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(amg_prolong, dim3(grid256(L.n)), dim3(256), 0, st, L.n, L.agg, C.x, L.x);
-    hipLaunchKernelGGL(amg_smooth, dim3(grid256(L.n)), dim3(256), 0, st, L.n, L.rp, L.ci, L.a, L.dinv, b, L.x, x);
-    return hipGetLastError();
-}
-
-hipError_t PressureAmg::vcycle(const double* b, double* x, hipStream_t st)
-{
-    return cycle(0, b, x, st);
-}
-
-// --------------------------------------------------------------- launchers
 #define OCPX_B_SWITCH(X)                                                                            \
     switch (B) {                                                                                    \
     X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14)                                     \
     default: return hipErrorInvalidValue;                                                           \
     }
 
+hipError_t PressureAmg::values(int B, const double* val, const double* dinv, double* d0, hipStream_t st)
+{
+    Level& L0 = lv_[0];
+    const unsigned nblk = (unsigned)((L0.n + 64 / B - 1) / (64 / B));
+#define X(N) case N: hipLaunchKernelGGL(cpr_columns<N>, dim3(nblk), dim3(64), 0, st, L0.n, L0.rp, val, dinv, d0, L0.a); break;
+    OCPX_B_SWITCH(X)
+#undef X
+    for (size_t l = 0; l < lv_.size(); l++) {
+        Level& L = lv_[l];
+        hipLaunchKernelGGL(amg_dinv, dim3(grid256(L.n)), dim3(256), 0, st, L.n, L.rp, L.a, L.dinv);
+        if (l + 1 < lv_.size()) {
+            Level& C = lv_[l + 1];
+            hipLaunchKernelGGL(amg_gather, dim3(grid256(C.nnz)), dim3(256), 0, st, C.nnz, L.gp, L.gs, L.a, C.a);
+            if (L.ne) hipLaunchKernelGGL(amg_sell, dim3(grid256(L.ne)), dim3(256), 0, st, L.ne, L.src, L.a, L.sa);
+        }
+    }
+    const Level& Lc = lv_.back();
+    if (Lc.n <= DENSE_MAX) {
+        hipLaunchKernelGGL(amg_dense_lu, dim3(1), dim3(64), 0, st, (int)Lc.n, Lc.rp, Lc.ci, Lc.a, lu_, piv_);
+        hipLaunchKernelGGL(amg_dense_inv, dim3(1), dim3(64), 0, st, (int)Lc.n, lu_, piv_, inv_);
+    }
+    return hipGetLastError();
+}
+
+hipError_t PressureAmg::small_cycle(double* x, hipStream_t st)
+{
+    SmallHier h{};
+    h.nl = (int)lv_.size() - 1 - small_;
+    h.nd = (int)lv_.back().n;
+    h.inv = inv_;
+    h.dinvd = lv_.back().dinv;
+    for (int k = 0; k < h.nl; k++) {
+        const Level& L = lv_[small_ + k];
+        h.lv[k] = SmallLevel{(int)L.n, (int)L.nc, (int)L.nq, L.off, L.row, L.sci, L.cagg, L.sa, L.dinv};
+    }
+    hipLaunchKernelGGL(amg_small, dim3(1), dim3(SM_THREADS), 0, st, h, lv_[small_].b, x);
+    return hipGetLastError();
+}
+
+// Level l with its right-hand side in b and its first sweep in x; the result
+// goes to xo, which is another array (a sweep reads its neighbours' x).
+hipError_t PressureAmg::cycle(int l, double* xo, hipStream_t st)
+{
+    Level& L = lv_[l];
+    if (l == small_) return small_cycle(xo, st);
+    if (l + 1 == (int)lv_.size()) {           // no dense level: a few sweeps
+        double *in = L.x, *out = L.r;
+        for (int k = 0; k < 9; k++) {
+            hipLaunchKernelGGL(amg_smooth, dim3(grid256(L.n)), dim3(256), 0, st, L.n, L.rp, L.ci, L.a, L.dinv, L.b, in, out);
+            std::swap(in, out);
+        }
+        if (in != xo) return hipMemcpyAsync(xo, in, (size_t)L.n * sizeof(double), hipMemcpyDeviceToDevice, st);
+        return hipGetLastError();
+    }
+    Level& C = lv_[l + 1];
+    hipLaunchKernelGGL(amg_down, dim3(grid256(L.nq)), dim3(256), 0, st, L.nq, L.nc, L.off, L.row, L.sci, L.sa, L.b,
+                       L.x, C.dinv, C.b, C.x);
+    hipError_t e = cycle(l + 1, C.r, st);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(amg_up, dim3(grid256(L.nq)), dim3(256), 0, st, L.nq, L.off, L.row, L.sci, L.cagg, L.sa, L.dinv,
+                       L.b, L.x, C.r, xo);
+    return hipGetLastError();
+}
+
+hipError_t PressureAmg::vcycle(double* x, hipStream_t st)
+{
+    return cycle(0, x, st);
+}
+
+// --------------------------------------------------------------- launchers
 hipError_t run_gs_color(int B, const int32_t* rows, int64_t nrows, const int64_t* rowptr, const int32_t* col,
                         const double* val, const double* dinv, const double* rhat, double* x, hipStream_t st)
 {
@@ -432,37 +722,91 @@ hipError_t run_gs_color(int B, const int32_t* rows, int64_t nrows, const int64_t
 #undef X
     return hipGetLastError();
 }
-#undef OCPX_B_SWITCH
 
-hipError_t run_mdot(const double* V, int64_t ldv, int m, const double* w, int64_t len, double* part, double* out,
-                    hipStream_t st)
+hipError_t run_cpr_resid(int B, const int64_t* rowptr, const int32_t* col, const double* d0, const double* px,
+                         const double* v, double* R, double* z, int64_t nb, hipStream_t st)
 {
-    if (m <= 0 || m > MD_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(mdot_part, dim3(MD_BLOCKS), dim3(MD_THREADS), 0, st, V, ldv, m, w, len, part);
-    hipLaunchKernelGGL(mdot_final, dim3(1), dim3(MD_THREADS), 0, st, m, part, out);
+    if (nb == 0) return hipSuccess;
+    const unsigned nblk = (unsigned)((nb + 64 / B - 1) / (64 / B));
+#define X(N) case N: hipLaunchKernelGGL(cpr_resid<N>, dim3(nblk), dim3(64), 0, st, rowptr, col, d0, px, v, R, z, nb); break;
+    OCPX_B_SWITCH(X)
+#undef X
     return hipGetLastError();
 }
 
-int mdot_scratch_len() { return MD_BLOCKS * MD_MAX; }
-
-hipError_t run_maxpy(double* w, const double* V, int64_t ldv, int m, const double* h, int64_t len, hipStream_t st)
+hipError_t run_cpr_half(int B, int which, const int32_t* rows, int64_t nrows, const int64_t* rowptr,
+                        const int32_t* col, const double* val, const double* dinv, const double* px,
+                        const double* v, double* R, double* z, double* w, hipStream_t st)
 {
-    if (m <= 0 || m > MD_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(maxpy, dim3(grid256(len)), dim3(256), 0, st, w, V, ldv, m, h, len);
+    if (nrows == 0) return hipSuccess;
+    const unsigned nblk = (unsigned)((nrows + 64 / B - 1) / (64 / B));
+#define X(N) case N: if (which) hipLaunchKernelGGL((cpr_half<N, true>), dim3(nblk), dim3(64), 0, st, rows, nrows, rowptr, col, val, dinv, px, v, R, z, w); \
+        else hipLaunchKernelGGL((cpr_half<N, false>), dim3(nblk), dim3(64), 0, st, rows, nrows, rowptr, col, val, dinv, px, v, R, z, w); break;
+    OCPX_B_SWITCH(X)
+#undef X
     return hipGetLastError();
 }
 
-hipError_t run_gather_p(int B, const double* v, double* p, int64_t n, hipStream_t st)
-{
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(gather_p, dim3(grid256(n)), dim3(256), 0, st, B, v, p, n);
-    return hipGetLastError();
-}
-
-hipError_t run_scatter_p(int B, const double* p, double* v, int64_t n, int64_t len, hipStream_t st)
+hipError_t run_fg_scale(int B, double* v, const double* w, const double* scale, double s, int64_t nb, int64_t len,
+                        const double* dinv0, double* pb, double* px0, hipStream_t st)
 {
     if (len == 0) return hipSuccess;
-    hipLaunchKernelGGL(scatter_p, dim3(grid256(len)), dim3(256), 0, st, B, p, v, n, len);
+#define X(N) case N: hipLaunchKernelGGL(fg_scale<N>, dim3(grid256(len)), dim3(256), 0, st, v, w, scale, s, nb, len, dinv0, pb, px0); break;
+    OCPX_B_SWITCH(X)
+#undef X
+    return hipGetLastError();
+}
+#undef OCPX_B_SWITCH
+
+int fg_scratch_len() { return FG_BLOCKS * 32; }
+
+static unsigned fg_blocks(int64_t len)
+{
+    const int64_t b = (len + FG_THREADS - 1) / FG_THREADS;
+    return (unsigned)(b < 1 ? 1 : (b > FG_BLOCKS ? FG_BLOCKS : b));
+}
+
+#define OCPX_M_SWITCH(X)                                                                            \
+    switch (m) {                                                                                    \
+    X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17)    \
+    X(18) X(19) X(20) X(21) X(22) X(23) X(24) X(25) X(26) X(27) X(28) X(29) X(30) X(31)             \
+    default: return hipErrorInvalidValue;                                                           \
+    }
+
+hipError_t run_fg_dot(const double* V, int64_t ldv, int m, const double* w, int64_t len, double* part, unsigned* done,
+                      double* h, double* host, hipStream_t st)
+{
+    static_assert(FG_MAX == 31, "the cases of OCPX_M_SWITCH");
+#define X(M) case M: hipLaunchKernelGGL(fg_dot<M>, dim3(fg_blocks(len)), dim3(FG_THREADS), 0, st, V, ldv, w, len, part, done, h, host); break;
+    OCPX_M_SWITCH(X)
+#undef X
+    return hipGetLastError();
+}
+
+hipError_t run_fg_orth(double* w, const double* V, int64_t ldv, int m, const double* h, int64_t len, double* part,
+                       unsigned* done, double* h2, hipStream_t st)
+{
+#define X(M) case M: hipLaunchKernelGGL(fg_orth<M>, dim3(fg_blocks(len)), dim3(FG_THREADS), 0, st, w, V, ldv, h, len, part, done, h2); break;
+    OCPX_M_SWITCH(X)
+#undef X
+    return hipGetLastError();
+}
+
+hipError_t run_fg_orth_norm(double* w, const double* V, int64_t ldv, int m, const double* h, const double* h2,
+                            int64_t len, double* part, unsigned* done, double* host, double* scale, hipStream_t st)
+{
+#define X(M) case M: hipLaunchKernelGGL(fg_orth_norm<M>, dim3(fg_blocks(len)), dim3(FG_THREADS), 0, st, w, V, ldv, h, h2, len, part, done, host, scale); break;
+    OCPX_M_SWITCH(X)
+#undef X
+    return hipGetLastError();
+}
+#undef OCPX_M_SWITCH
+
+hipError_t run_fg_axpy(double* x, const double* Z, int64_t ldz, int m, const FgCoef& y, int64_t len, hipStream_t st)
+{
+    if (len == 0) return hipSuccess;
+    if (m < 0 || m > 32) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(fg_axpy, dim3(grid256(len)), dim3(256), 0, st, x, Z, ldz, m, y, len);
     return hipGetLastError();
 }
 

@@ -20,7 +20,9 @@
 //    coarsest level.
 //  * the second stage: one multicolour block Gauss-Seidel sweep on the
 //    decoupled system (whose diagonal blocks are the identity), colours
-//    from a greedy colouring of the block graph.
+//    from a greedy colouring of the block graph.  With two colours (any
+//    Cartesian grid) the sweep and the operator that follows it share one
+//    read of the matrix (cpr.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -47,12 +49,18 @@ public:
     int64_t rows(int l) const { return lv_[l].n; }
 
     // Level matrices of the current system: val the bulk BSR (B x B blocks,
-    // row-major), dinv the inverses of its diagonal blocks.
-    hipError_t values(int B, const double* val, const double* dinv, hipStream_t st);
-    // x = one V-cycle applied to b (level-0 vectors of n doubles)
-    hipError_t vcycle(const double* b, double* x, hipStream_t st);
+    // row-major), dinv the inverses of its diagonal blocks, d0 [nnzb][B] receives
+    // column 0 of every decoupled block D_i^{-1} A_ij.
+    hipError_t values(int B, const double* val, const double* dinv, double* d0, hipStream_t st);
+    // x = one V-cycle applied to b; b is already in place: level0_b() and
+    // level0_x() (= OMEGA Dinv b) hold the level-0 right-hand side and its first sweep
+    hipError_t vcycle(double* x, hipStream_t st);
+    double* level0_b() { return lv_[0].b; }
+    double* level0_x() { return lv_[0].x; }
+    const double* level0_dinv() const { return lv_[0].dinv; }
 
     static constexpr int DENSE_MAX = 64;     // the coarsest level is solved densely up to this size
+    static constexpr double OMEGA = 2.0 / 3.0;   // weighted-Jacobi smoother
 
 private:
     struct Level {
@@ -61,32 +69,55 @@ private:
         int32_t* ci = nullptr;
         double *a = nullptr, *dinv = nullptr, *b = nullptr, *x = nullptr, *r = nullptr;
         // to the next level (all but the last)
-        int32_t* agg = nullptr;              // [n] coarse row of each row
         int64_t *gp = nullptr, *gs = nullptr;   // coarse slot s = sum of a[gs[gp[s] .. gp[s+1])]
-        int64_t* mp = nullptr;               // coarse row I: fine rows mi[mp[I] .. mp[I+1])
-        int32_t* mi = nullptr;
+        // the level's matrix in V-cycle order (amg::Sell); ne entries
+        int64_t nc = 0, nq = 0, ne = 0;
+        int64_t* off = nullptr;
+        int32_t *row = nullptr, *sci = nullptr, *cagg = nullptr, *src = nullptr;
+        double* sa = nullptr;
     };
     std::vector<Level> lv_;
-    double* lu_ = nullptr;                   // dense LU of the coarsest level (DENSE_MAX^2)
+    int small_ = -1;                         // first level of the one-workgroup part of the cycle, -1 none
+    double *lu_ = nullptr, *inv_ = nullptr;  // dense LU and inverse of the coarsest level (DENSE_MAX^2)
     int32_t* piv_ = nullptr;
-    const int64_t* rp0_ = nullptr;           // level-0 pattern (device, the bulk BSR's)
     std::vector<void*> mem_;
     template <class T>
     int dev(T** p, size_t count, const T* host, std::string& err);
-    hipError_t cycle(int l, const double* b, double* x, hipStream_t st);
+    hipError_t cycle(int l, double* x, hipStream_t st);
+    hipError_t small_cycle(double* x, hipStream_t st);
 };
 
 // x_i = rhat_i - Dinv_i sum_{j != i} A_ij x_j for the rows of one colour
 hipError_t run_gs_color(int B, const int32_t* rows, int64_t nrows, const int64_t* rowptr, const int32_t* col,
                         const double* val, const double* dinv, const double* rhat, double* x, hipStream_t st);
-// out[k] = V_k . w for k < m (V: m vectors of len doubles, stride ldv)
-hipError_t run_mdot(const double* V, int64_t ldv, int m, const double* w, int64_t len, double* part, double* out,
-                    hipStream_t st);
-int mdot_scratch_len();
-// w += sum_{k < m} h[k] V_k (h on the device, m <= 32)
-hipError_t run_maxpy(double* w, const double* V, int64_t ldv, int m, const double* h, int64_t len, hipStream_t st);
-// the pressure entries of a block vector and back: p[i] = v[i B], v = 0 except v[i B] = p[i]
-hipError_t run_gather_p(int B, const double* v, double* p, int64_t n, hipStream_t st);
-hipError_t run_scatter_p(int B, const double* p, double* v, int64_t n, int64_t len, hipStream_t st);
+
+// ---- FGMRES pieces on vectors of len doubles (the last block of each
+// reduction sums the partials in block order, so results have the same bits on
+// every run).  part: fg_scratch_len() doubles; done: one word, 0 before the
+// first call and after every call.
+int fg_scratch_len();
+// h[k] = V_k . w for k < m (V: m vectors, stride ldv; m <= 31); host (pinned, may be null) gets a copy
+hipError_t run_fg_dot(const double* V, int64_t ldv, int m, const double* w, int64_t len, double* part, unsigned* done,
+                      double* h, double* host, hipStream_t st);
+// w -= sum h[k] V_k, then h2[k] = V_k . w
+hipError_t run_fg_orth(double* w, const double* V, int64_t ldv, int m, const double* h, int64_t len, double* part,
+                       unsigned* done, double* h2, hipStream_t st);
+// w -= sum h2[k] V_k; host[k] = h[k] + h2[k], host[m] = w . w; *scale = 1 / |w|
+hipError_t run_fg_orth_norm(double* w, const double* V, int64_t ldv, int m, const double* h, const double* h2,
+                            int64_t len, double* part, unsigned* done, double* host, double* scale, hipStream_t st);
+// v = w * (scale ? *scale : s); for the nb bulk rows pb = v's pressure entries and px0 = OMEGA dinv0 pb
+hipError_t run_fg_scale(int B, double* v, const double* w, const double* scale, double s, int64_t nb, int64_t len,
+                        const double* dinv0, double* pb, double* px0, hipStream_t st);
+struct FgCoef { double y[32]; };
+// x += sum_{k < m} y[k] Z_k
+hipError_t run_fg_axpy(double* x, const double* Z, int64_t ldz, int m, const FgCoef& y, int64_t len, hipStream_t st);
+
+// R = v - Dinv J x1 and z = R + x1 on the bulk rows, x1 the pressure correction px (0 in the other entries)
+hipError_t run_cpr_resid(int B, const int64_t* rowptr, const int32_t* col, const double* d0, const double* px,
+                         const double* v, double* R, double* z, int64_t nb, hipStream_t st);
+// the second and the first colour of a two-colour graph (which = 1, 0), see cpr.hip
+hipError_t run_cpr_half(int B, int which, const int32_t* rows, int64_t nrows, const int64_t* rowptr,
+                        const int32_t* col, const double* val, const double* dinv, const double* px,
+                        const double* v, double* R, double* z, double* w, hipStream_t st);
 
 }  // namespace ocpx

@@ -125,8 +125,10 @@ struct ocpx_ctx {
     std::vector<int32_t> gs_cptr;        // colour lists of the block Gauss-Seidel stage
     int32_t* gs_rows = nullptr;
     double *fg_V = nullptr, *fg_Z = nullptr, *fg_w = nullptr, *fg_t = nullptr, *fg_x1 = nullptr;
-    double *fg_r2 = nullptr, *fg_pb = nullptr, *fg_px = nullptr, *fg_h = nullptr, *fg_part = nullptr;
-    double* fg_out = nullptr;
+    double *fg_r2 = nullptr, *fg_px = nullptr, *fg_h = nullptr, *fg_part = nullptr;
+    double* fg_d0 = nullptr;             // [nnzb][b] column 0 of every decoupled block
+    unsigned* fg_done = nullptr;         // blocks of the current reduction that are done
+    double* fg_host = nullptr;           // pinned: the Hessenberg column and the norm of each iteration
     int64_t fg_cap = 0;
     // timing
     bool timing = false;
@@ -774,6 +776,7 @@ void ocpx_ctx_destroy(ocpx_ctx* c)
     for (auto& t : c->tacc)
         for (auto& p : t.pending) { hipEventDestroy(p.first); hipEventDestroy(p.second); }
     for (void* p : c->allocs) hipFree(p);
+    if (c->fg_host) hipHostFree(c->fg_host);
     if (c->own_stream) hipStreamDestroy(c->st);
     if (c->st2) hipStreamDestroy(c->st2);
     if (c->ev_fork) hipEventDestroy(c->ev_fork);
@@ -1401,7 +1404,9 @@ int cpr_setup(ocpx_ctx* c)
 // multicolour block Gauss-Seidel sweep on the remaining residual.  Classical
 // Gram-Schmidt with one reorthogonalisation; stops on the decoupled
 // ||r|| / ||b||, as FASP's stop_type 1 on the decoupled system.  x0 = 0,
-// the solution in c->sol.
+// the solution in c->sol.  The host waits once per iteration, for the
+// Hessenberg column; the products and updates before it pass their scalars on
+// the device.
 int fgmres_cpr(ocpx_ctx* c, const double* rhs, int64_t len, int32_t nwj, double rtol, int32_t maxit, int& it,
                double& res, bool& conv)
 {
@@ -1413,21 +1418,26 @@ int fgmres_cpr(ocpx_ctx* c, const double* rhs, int64_t len, int32_t nwj, double 
     if (rc) return rc;
     if (c->fg_cap < len) {
         for (double** q : {&c->fg_V, &c->fg_Z, &c->fg_w, &c->fg_t, &c->fg_x1, &c->fg_r2}) { dfree(c, *q); *q = nullptr; }
+        c->fg_cap = 0;
         if ((rc = dalloc(c, &c->fg_V, (size_t)(M + 1) * len)) || (rc = dalloc(c, &c->fg_Z, (size_t)M * len)) ||
             (rc = dalloc(c, &c->fg_w, (size_t)len)) || (rc = dalloc(c, &c->fg_t, (size_t)len)) ||
             (rc = dalloc(c, &c->fg_x1, (size_t)len)) || (rc = dalloc(c, &c->fg_r2, (size_t)len)))
             return rc;
         c->fg_cap = len;
     }
-    if (!c->fg_pb) {
-        if ((rc = dalloc(c, &c->fg_pb, (size_t)nb)) || (rc = dalloc(c, &c->fg_px, (size_t)nb)) ||
-            (rc = dalloc(c, &c->fg_h, 64)) || (rc = dalloc(c, &c->fg_part, (size_t)mdot_scratch_len())) ||
-            (rc = dalloc(c, &c->fg_out, 64)))
+    if (!c->fg_host) {
+        if ((rc = dalloc(c, &c->fg_px, (size_t)nb)) || (rc = dalloc(c, &c->fg_d0, (size_t)c->nnzb * B)) ||
+            (rc = dalloc(c, &c->fg_h, 128)) || (rc = dalloc(c, &c->fg_part, (size_t)fg_scratch_len())) ||
+            (rc = dalloc(c, &c->fg_done, 1)))
             return rc;
+        HIPCHK(c, hipHostMalloc((void**)&c->fg_host, 64 * sizeof(double), hipHostMallocDefault));
     }
     const BsrIO io = bsr_io(c);
     const WellIO wio = well_io(c);
-    double *V = c->fg_V, *Z = c->fg_Z, *w = c->fg_w, *t = c->fg_t, *x = c->sol;
+    double *V = c->fg_V, *Z = c->fg_Z, *w = c->fg_w, *t = c->fg_t, *R = c->fg_r2, *px = c->fg_px, *x = c->sol;
+    double *dh = c->fg_h, *dh2 = c->fg_h + 32, *dscale = c->fg_h + 64;
+    volatile double* host = c->fg_host;
+    PressureAmg& amg = *c->amg;
     // y = D^{-1} J x
     auto aop = [&](const double* in, double* out) -> int {
         {
@@ -1439,46 +1449,49 @@ int fgmres_cpr(ocpx_ctx* c, const double* rhs, int64_t len, int32_t nwj, double 
         if (nwj) HIPCHK(c, run_bsr_spmv(B, nullptr, nullptr, c->dinv_w, t + nb * B, out + nb * B, nwj, st));
         return OCPX_OK;
     };
-    // z = M^{-1} v
-    auto precond = [&](const double* v, double* z) -> int {
-        HIPCHK(c, run_gather_p(B, v, c->fg_pb, nb, st));
-        HIPCHK(c, c->amg->vcycle(c->fg_pb, c->fg_px, st));
-        HIPCHK(c, run_scatter_p(B, c->fg_px, c->fg_x1, nb, len, st));
-        int rr = aop(c->fg_x1, c->fg_r2);
-        if (rr) return rr;
-        HIPCHK(c, run_axpbypcz(c->fg_r2, v, -1.0, c->fg_r2, 0, nullptr, len, st));    // r2 = v - A x1
-        // z = r2 on every row, then the colours of the bulk rows in turn
-        // (rows of one colour read only rows of other colours)
-        HIPCHK(c, run_axpbypcz(z, nullptr, 0, nullptr, 0, nullptr, nb * B, st));
-        if (nwj) HIPCHK(c, run_axpbypcz(z + nb * B, c->fg_r2 + nb * B, 0, nullptr, 0, nullptr, (int64_t)nwj * B, st));
+    auto colour = [&](size_t k) { return c->gs_rows + c->gs_cptr[k]; };
+    auto ncolour = [&](size_t k) { return (int64_t)(c->gs_cptr[k + 1] - c->gs_cptr[k]); };
+    // z = M^{-1} v and w = D^{-1} J z; v's pressures are in the AMG's level 0
+    auto precond_op = [&](const double* v, double* z) -> int {
+        HIPCHK(c, amg.vcycle(px, st));
+        HIPCHK(c, run_cpr_resid(B, io.rowptr, io.colind, c->fg_d0, px, v, R, z, nb, st));
+        if (nwj) HIPCHK(c, run_well_resid(wio, B, nb, c->dinv_w, px, v, z, st));
+        if (c->gs_cptr.size() == 3) {            // two colours: the sweep and the operator in one read of the matrix
+            HIPCHK(c, run_cpr_half(B, 1, colour(1), ncolour(1), io.rowptr, io.colind, io.val, c->dinv, px, v, R, z, w, st));
+            HIPCHK(c, run_cpr_half(B, 0, colour(0), ncolour(0), io.rowptr, io.colind, io.val, c->dinv, px, v, R, z, w, st));
+            if (nwj) HIPCHK(c, run_well_dapply(wio, B, nb, c->dinv, c->dinv_w, z, w, st));
+            return OCPX_OK;
+        }
+        // the colours of the bulk rows in turn (rows of one colour read only
+        // rows of other colours), then the operator; z is R + x1 here, so the
+        // sweep's change of R is added to it
+        double* g = c->fg_x1;
+        HIPCHK(c, run_axpbypcz(g, nullptr, 0, nullptr, 0, nullptr, nb * B, st));
         for (size_t k = 0; k + 1 < c->gs_cptr.size(); k++)
-            HIPCHK(c, run_gs_color(B, c->gs_rows + c->gs_cptr[k], c->gs_cptr[k + 1] - c->gs_cptr[k], io.rowptr,
-                                   io.colind, io.val, c->dinv, c->fg_r2, z, st));
-        HIPCHK(c, run_axpbypcz(z, z, 1.0, c->fg_x1, 0, nullptr, len, st));
-        return OCPX_OK;
+            HIPCHK(c, run_gs_color(B, colour(k), ncolour(k), io.rowptr, io.colind, io.val, c->dinv, R, g, st));
+        HIPCHK(c, run_axpbypcz(R, g, -1.0, R, 0, nullptr, nb * B, st));
+        HIPCHK(c, run_axpbypcz(z, z, 1.0, R, 0, nullptr, nb * B, st));
+        return aop(z, w);
     };
-    auto dots = [&](const double* Vb, int m, const double* vec, double* out) -> int {
-        HIPCHK(c, run_mdot(Vb, len, m, vec, len, c->fg_part, c->fg_out, st));
-        HIPCHK(c, hipMemcpyAsync(out, c->fg_out, (size_t)m * sizeof(double), hipMemcpyDeviceToHost, st));
-        HIPCHK(c, hipStreamSynchronize(st));
-        return OCPX_OK;
-    };
-    HIPCHK(c, c->amg->values(B, io.val, c->dinv, st));
-    // b = D^{-1} rhs into V_0's slot for now; x = 0
-    double* bh = c->fg_r2;
-    HIPCHK(c, run_bsr_spmv(B, nullptr, nullptr, c->dinv, rhs, V, nb, st));
-    if (nwj) HIPCHK(c, run_bsr_spmv(B, nullptr, nullptr, c->dinv_w, rhs + nb * B, V + nb * B, nwj, st));
+    HIPCHK(c, amg.values(B, io.val, c->dinv, c->fg_d0, st));
+    // b = D^{-1} rhs; x = 0
+    HIPCHK(c, run_bsr_spmv(B, nullptr, nullptr, c->dinv, rhs, w, nb, st));
+    if (nwj) HIPCHK(c, run_bsr_spmv(B, nullptr, nullptr, c->dinv_w, rhs + nb * B, w + nb * B, nwj, st));
     HIPCHK(c, run_axpbypcz(x, nullptr, 0, nullptr, 0, nullptr, len, st));
-    double bb = 0;
-    if ((rc = dots(V, 1, V, &bb))) return rc;
-    const double bnorm = std::sqrt(bb);
+    auto norm_w = [&](double& out) -> int {
+        HIPCHK(c, run_fg_dot(w, len, 1, w, len, c->fg_part, c->fg_done, dh, c->fg_host, st));
+        HIPCHK(c, hipStreamSynchronize(st));
+        out = std::sqrt(host[0]);
+        return OCPX_OK;
+    };
+    double bnorm = 0;
+    if ((rc = norm_w(bnorm))) return rc;
     double beta = bnorm;
     it = 0;
     res = 0;
     conv = bnorm == 0;
-    std::vector<double> H((M + 1) * M), cs(M), sn(M), g(M + 1), y(M), h(M + 1), h2(M + 1);
+    std::vector<double> H((M + 1) * M), cs(M), sn(M), g(M + 1), y(M);
     while (!conv && it < maxit && std::isfinite(beta) && beta > 0) {
-        HIPCHK(c, run_axpbypcz(V, nullptr, 1.0 / beta, V, 0, nullptr, len, st));        // V_0 = r / beta
         std::fill(g.begin(), g.end(), 0.0);
         g[0] = beta;
         int k = 0;
@@ -1486,21 +1499,16 @@ int fgmres_cpr(ocpx_ctx* c, const double* rhs, int64_t len, int32_t nwj, double 
         for (int j = 0; j < M && it < maxit; j++) {
             double* Vj = V + (size_t)j * len;
             double* Zj = Z + (size_t)j * len;
-            if ((rc = precond(Vj, Zj)) || (rc = aop(Zj, w))) return rc;
-            if ((rc = dots(V, j + 1, w, h.data()))) return rc;
-            for (int i = 0; i <= j; i++) h2[i] = -h[i];
-            HIPCHK(c, hipMemcpyAsync(c->fg_h, h2.data(), (size_t)(j + 1) * 8, hipMemcpyHostToDevice, st));
-            HIPCHK(c, run_maxpy(w, V, len, j + 1, c->fg_h, len, st));
-            if ((rc = dots(V, j + 1, w, h2.data()))) return rc;
-            for (int i = 0; i <= j; i++) { h[i] += h2[i]; h2[i] = -h2[i]; }
-            HIPCHK(c, hipMemcpyAsync(c->fg_h, h2.data(), (size_t)(j + 1) * 8, hipMemcpyHostToDevice, st));
-            HIPCHK(c, run_maxpy(w, V, len, j + 1, c->fg_h, len, st));
-            double ww = 0;
-            HIPCHK(c, run_dot(w, w, len, c->dpart, c->dout, st));
-            HIPCHK(c, hipMemcpyAsync(&ww, c->dout, sizeof(double), hipMemcpyDeviceToHost, st));
+            // V_j = r / beta or w / |w|, w the last orthogonalised vector
+            HIPCHK(c, run_fg_scale(B, Vj, w, j ? dscale : nullptr, 1.0 / beta, nb, len, amg.level0_dinv(), amg.level0_b(),
+                                   amg.level0_x(), st));
+            if ((rc = precond_op(Vj, Zj))) return rc;
+            HIPCHK(c, run_fg_dot(V, len, j + 1, w, len, c->fg_part, c->fg_done, dh, nullptr, st));
+            HIPCHK(c, run_fg_orth(w, V, len, j + 1, dh, len, c->fg_part, c->fg_done, dh2, st));
+            HIPCHK(c, run_fg_orth_norm(w, V, len, j + 1, dh, dh2, len, c->fg_part, c->fg_done, c->fg_host, dscale, st));
             HIPCHK(c, hipStreamSynchronize(st));
-            const double hn = std::sqrt(ww);
-            for (int i = 0; i <= j; i++) H[i * M + j] = h[i];
+            const double hn = std::sqrt(host[j + 1]);
+            for (int i = 0; i <= j; i++) H[i * M + j] = host[i];
             H[(j + 1) * M + j] = hn;
             for (int i = 0; i < j; i++) {             // earlier rotations
                 const double a = H[i * M + j], b2 = H[(i + 1) * M + j];
@@ -1520,23 +1528,21 @@ int fgmres_cpr(ocpx_ctx* c, const double* rhs, int64_t len, int32_t nwj, double 
             res = std::fabs(g[j + 1]) / bnorm;
             if (!std::isfinite(res)) return fail(c, OCPX_E_HIP, "FGMRES: non-finite residual");
             if (res < rtol || hn == 0) { stop = true; break; }
-            HIPCHK(c, run_axpbypcz(V + (size_t)(j + 1) * len, nullptr, 1.0 / hn, w, 0, nullptr, len, st));
         }
         for (int i = k - 1; i >= 0; i--) {           // H y = g, upper triangular
             double v = g[i];
             for (int q = i + 1; q < k; q++) v -= H[i * M + q] * y[q];
             y[i] = H[i * M + i] != 0 ? v / H[i * M + i] : 0.0;
         }
-        HIPCHK(c, hipMemcpyAsync(c->fg_h, y.data(), (size_t)k * 8, hipMemcpyHostToDevice, st));
-        HIPCHK(c, run_maxpy(x, Z, len, k, c->fg_h, len, st));
-        // the true decoupled residual: V_0 = D^{-1} rhs - D^{-1} J x
-        if ((rc = aop(x, w))) return rc;
-        HIPCHK(c, run_bsr_spmv(B, nullptr, nullptr, c->dinv, rhs, bh, nb, st));
-        if (nwj) HIPCHK(c, run_bsr_spmv(B, nullptr, nullptr, c->dinv_w, rhs + nb * B, bh + nb * B, nwj, st));
-        HIPCHK(c, run_axpbypcz(V, bh, -1.0, w, 0, nullptr, len, st));
-        double rr2 = 0;
-        if ((rc = dots(V, 1, V, &rr2))) return rc;
-        beta = std::sqrt(rr2);
+        FgCoef co{};
+        for (int i = 0; i < k; i++) co.y[i] = y[i];
+        HIPCHK(c, run_fg_axpy(x, Z, len, k, co, len, st));
+        // the true decoupled residual: w = D^{-1} rhs - D^{-1} J x
+        if ((rc = aop(x, R))) return rc;
+        HIPCHK(c, run_bsr_spmv(B, nullptr, nullptr, c->dinv, rhs, w, nb, st));
+        if (nwj) HIPCHK(c, run_bsr_spmv(B, nullptr, nullptr, c->dinv_w, rhs + nb * B, w + nb * B, nwj, st));
+        HIPCHK(c, run_axpbypcz(w, w, -1.0, R, 0, nullptr, len, st));
+        if ((rc = norm_w(beta))) return rc;
         res = beta / bnorm;
         if (res < rtol) conv = true;
         if (stop && !conv && k == 0) break;

@@ -234,6 +234,12 @@ hipError_t run_well_terms(int nc, const CellIO& c, const BsrIO& bsr, const WellI
                           double* resAbs, hipStream_t st);
 // the well rows and columns of y = A x after the bulk bsr_spmv (x, y of length (nb + nwell) * B)
 hipError_t run_well_spmv(const WellIO& w, int B, int64_t nb, const double* x, double* y, hipStream_t st);
+// the well rows of z = v - Dinv J x1, x1 the pressure correction px on the bulk rows
+hipError_t run_well_resid(const WellIO& w, int B, int64_t nb, const double* dinv_w, const double* px, const double* v,
+                          double* z, hipStream_t st);
+// the wells' part of y = D^{-1} J z on top of the bulk rows' own part in y
+hipError_t run_well_dapply(const WellIO& w, int B, int64_t nb, const double* dinv, const double* dinv_w,
+                           const double* z, double* y, hipStream_t st);
 // bhp += u[(nb + w) * B] for every well (device copy of the wells)
 hipError_t run_well_bhp_update(ocpx_well* wells, int32_t nwell, int B, int64_t nb, const double* u, hipStream_t st);
 hipError_t run_get_solution(int nc, double* P, double* Ni, double* S, double* xij,

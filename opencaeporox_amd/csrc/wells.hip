@@ -270,6 +270,72 @@ __global__ void __launch_bounds__(64) well_spmv(WellIO w, int B, int64_t nb, con
     }
 }
 
+// sum over a well's perforations of row 0 of its (w, n) blocks times the cell's
+// entries, 64 lanes; with P, of the pressure entries of a pressure vector only
+template <bool P>
+__device__ __forceinline__ double well_row0(const WellIO& w, const ocpx_well& W, int B, const double* x, double* part)
+{
+    const int lane = threadIdx.x;
+    double c0 = 0;
+    for (int p = W.perf0 + lane; p < W.perf0 + W.nperf; p += 64) {
+        const int64_t n = w.cell[p];
+        if constexpr (P) c0 += w.Cwn[(size_t)p * B] * x[n];
+        else for (int col = 0; col < B; col++) c0 += w.Cwn[(size_t)p * B + col] * x[(size_t)n * B + col];
+    }
+    part[lane] = c0;
+    __syncthreads();
+    for (int s = 32; s > 0; s >>= 1) {
+        if (lane < s) part[lane] += part[lane + s];
+        __syncthreads();
+    }
+    return part[0];
+}
+
+// The well rows of z = v - Dinv J x1 for a pressure correction x1 (px; 0 in the
+// well rows), one workgroup per well
+__global__ void __launch_bounds__(64) well_resid(WellIO w, int B, int64_t nb, const double* __restrict__ dinv_w,
+                                                 const double* __restrict__ px, const double* __restrict__ v,
+                                                 double* __restrict__ z)
+{
+    __shared__ double part[64];
+    const int iw = blockIdx.x, lane = threadIdx.x;
+    const double c = well_row0<true>(w, w.wells[iw], B, px, part);
+    const size_t o = (size_t)(nb + iw) * B + lane;
+    if (lane < B) z[o] = v[o] - dinv_w[((size_t)iw * B + lane) * B] * c;
+}
+
+// The wells' part of y = D^{-1} J z where y holds the bulk rows' own part:
+// y[bulk] += Dinv_n Bnw z[well] (workgroups 0 .. nucell - 1) and the well rows,
+// whose diagonal block's product is z itself (one workgroup per well)
+__global__ void __launch_bounds__(64) well_dapply(WellIO w, int B, int64_t nb, const double* __restrict__ dinv,
+                                                  const double* __restrict__ dinv_w, const double* __restrict__ z,
+                                                  double* __restrict__ y)
+{
+    __shared__ double part[64];
+    const int lane = threadIdx.x, g = blockIdx.x;
+    if (g < w.nucell) {                                              // uniform per workgroup
+        const int64_t n = w.ucell[g];
+        double acc = 0;
+        if (lane < B)
+            for (int k = w.uptr[g]; k < w.uptr[g + 1]; k++) {
+                const int p = w.uperf[k];
+                acc += w.Bnw[(size_t)p * B + lane] * z[(size_t)(nb + w.pwell[p]) * B];
+            }
+        part[lane] = acc;
+        __syncthreads();
+        if (lane < B) {
+            double t = y[(size_t)n * B + lane];
+            for (int c = 0; c < B; c++) t += dinv[((size_t)n * B + lane) * B + c] * part[c];
+            y[(size_t)n * B + lane] = t;
+        }
+        return;
+    }
+    const int iw = g - w.nucell;
+    const double c = well_row0<false>(w, w.wells[iw], B, z, part);
+    const size_t o = (size_t)(nb + iw) * B + lane;
+    if (lane < B) y[o] = z[o] + dinv_w[((size_t)iw * B + lane) * B] * c;
+}
+
 // PeacemanWellIsoT::GetSolutionFIM (src/WellPeaceman.cpp:1198-1204): bhp += u of the well row
 __global__ void __launch_bounds__(64) well_bhp_update(ocpx_well* wells, int32_t nwell, int B, int64_t nb,
                                                       const double* __restrict__ u)
@@ -282,6 +348,22 @@ hipError_t run_well_spmv(const WellIO& w, int B, int64_t nb, const double* x, do
 {
     if (w.nwell == 0) return hipSuccess;
     hipLaunchKernelGGL(well_spmv, dim3(w.nucell + w.nwell), dim3(64), 0, st, w, B, nb, x, y);
+    return hipGetLastError();
+}
+
+hipError_t run_well_resid(const WellIO& w, int B, int64_t nb, const double* dinv_w, const double* px, const double* v,
+                          double* z, hipStream_t st)
+{
+    if (w.nwell == 0) return hipSuccess;
+    hipLaunchKernelGGL(well_resid, dim3(w.nwell), dim3(64), 0, st, w, B, nb, dinv_w, px, v, z);
+    return hipGetLastError();
+}
+
+hipError_t run_well_dapply(const WellIO& w, int B, int64_t nb, const double* dinv, const double* dinv_w,
+                           const double* z, double* y, hipStream_t st)
+{
+    if (w.nwell == 0) return hipSuccess;
+    hipLaunchKernelGGL(well_dapply, dim3(w.nucell + w.nwell), dim3(64), 0, st, w, B, nb, dinv, dinv_w, z, y);
     return hipGetLastError();
 }
 

@@ -26,6 +26,7 @@ HARNESS = r'''
 using namespace ocpx;
 static amg::Graph G, GC;
 static amg::LevelMaps M;
+static amg::Sell S;
 extern "C" {
 void layout(int64_t nb, int64_t nconn, const int32_t* cb, const int32_t* ce, int64_t* rp, int32_t* col,
             int32_t* ts, int32_t* nbc) { bsr_layout(nb, nconn, cb, ce, rp, col, ts, nbc); }
@@ -47,6 +48,18 @@ void fetch(int64_t* crp, int32_t* cci, double* cw, int32_t* agg, int64_t* gp, in
     for (size_t k = 0; k < M.gs.size(); k++) gs[k] = M.gs[k];
     for (size_t k = 0; k < M.mp.size(); k++) mp[k] = M.mp[k];
     for (size_t k = 0; k < M.mi.size(); k++) mi[k] = M.mi[k];
+}
+int64_t sell_sizes(int64_t* out)
+{
+    amg::sell_layout(G, M, GC.n, S);
+    out[0] = (int64_t)S.row.size(); out[1] = (int64_t)S.off.size(); out[2] = (int64_t)S.ci.size();
+    return 0;
+}
+void sell_fetch(int64_t* off, int32_t* row, int32_t* ci, int32_t* cagg, int32_t* src)
+{
+    for (size_t k = 0; k < S.off.size(); k++) off[k] = S.off[k];
+    for (size_t k = 0; k < S.row.size(); k++) row[k] = S.row[k];
+    for (size_t k = 0; k < S.ci.size(); k++) { ci[k] = S.ci[k]; cagg[k] = S.cagg[k]; src[k] = S.src[k]; }
 }
 int64_t colors(int64_t n, const int64_t* rp, const int32_t* ci, int32_t* cptr, int32_t* rows)
 {
@@ -158,3 +171,42 @@ def test_colouring(lib):
     frow = np.repeat(np.arange(n), np.diff(rp))
     off = frow != ci
     assert np.all(color[frow[off]] != color[ci[off]])
+
+
+@pytest.mark.parametrize("dims", [(5, 4, 4), (17, 13, 7), (40, 30, 20)])
+def test_sliced_layout(lib, dims):
+    """The V-cycle's walk of a level: every CSR slot appears once, at a
+    position of its own row, with its column and that column's aggregate; the
+    positions 4 I .. 4 I + 3 are aggregate I's members; padding reads valid
+    rows."""
+    n, rp, ci, w = _level0(lib, dims)
+    while n > DENSE_MAX:
+        if not lib.coarsen(C.c_int64(n), _p(rp), _p(ci), _p(w)):
+            break
+        sz, ss = np.zeros(2, np.int64), np.zeros(3, np.int64)
+        lib.sizes(_p(sz))
+        nc, nnzc = int(sz[0]), int(sz[1])
+        crp, cci, cw = np.zeros(nc + 1, np.int64), np.zeros(nnzc, np.int32), np.zeros(nnzc)
+        agg, mi = np.zeros(n, np.int32), np.zeros(n, np.int32)
+        gp, gs, mp = np.zeros(nnzc + 1, np.int64), np.zeros(rp[-1], np.int64), np.zeros(nc + 1, np.int64)
+        lib.fetch(_p(crp), _p(cci), _p(cw), _p(agg), _p(gp), _p(gs), _p(mp), _p(mi))
+        lib.sell_sizes(_p(ss))
+        nq, noff, ne = (int(v) for v in ss)
+        off, row = np.zeros(noff, np.int64), np.zeros(nq, np.int32)
+        sci, cagg, src = (np.zeros(ne, np.int32) for _ in range(3))
+        lib.sell_fetch(_p(off), _p(row), _p(sci), _p(cagg), _p(src))
+        assert nq % 64 == 0 and 4 * nc <= nq < 4 * nc + 64 and noff == nq // 64 + 1
+        assert off[0] == 0 and off[-1] == ne and np.all(np.diff(off) % 64 == 0)
+        q = np.arange(nq)
+        held = row >= 0
+        assert np.array_equal(np.sort(row[held]), np.arange(n))
+        assert np.array_equal(agg[row[held]], q[held] // 4)
+        # entry -> position: lane of the slice it lies in
+        e = np.arange(ne)
+        pos = (np.searchsorted(off, e, side="right") - 1) * 64 + (e - off[np.searchsorted(off, e, side="right") - 1]) % 64
+        real = src >= 0
+        assert np.array_equal(np.sort(src[real]), np.arange(rp[-1]))
+        frow = np.repeat(np.arange(n), np.diff(rp))
+        assert np.array_equal(row[pos[real]], frow[src[real]]) and np.array_equal(sci[real], ci[src[real]])
+        assert sci.min() >= 0 and sci.max() < n and np.array_equal(cagg, agg[sci])
+        n, rp, ci, w = nc, crp, cci, cw
