@@ -13,6 +13,7 @@
 #include "amg_layout.hpp"
 #include "cpr.hpp"
 #include "ocpx_dev.hpp"
+#include "ocpx_kernels.hpp"
 
 namespace ocpx {
 
@@ -134,7 +135,13 @@ __global__ void __launch_bounds__(256) amg_down(int64_t nq, int64_t nc, const in
     if (i >= 0) {
         r = b[i];
         const int64_t e1 = off[(q >> 6) + 1];
-        for (int64_t e = off[q >> 6] + (q & 63); e < e1; e += 64) r -= a[e] * x[ci[e]];
+        int64_t e = off[q >> 6] + (q & 63);
+        for (; e + 192 < e1; e += 256) {            // four entries in flight
+            double av[4], xv[4];
+            UNROLL for (int u = 0; u < 4; u++) { av[u] = a[e + 64 * u]; xv[u] = x[ci[e + 64 * u]]; }
+            UNROLL for (int u = 0; u < 4; u++) r -= av[u] * xv[u];
+        }
+        for (; e < e1; e += 64) r -= a[e] * x[ci[e]];
     }
     r += __shfl_xor(r, 1);
     r += __shfl_xor(r, 2);
@@ -160,7 +167,13 @@ __global__ void __launch_bounds__(256) amg_up(int64_t nq, const int64_t* __restr
     if (i < 0) return;
     double r = b[i];
     const int64_t e1 = off[(q >> 6) + 1];
-    for (int64_t e = off[q >> 6] + (q & 63); e < e1; e += 64) r -= a[e] * (x[ci[e]] + xc[cagg[e]]);
+    int64_t e = off[q >> 6] + (q & 63);
+    for (; e + 192 < e1; e += 256) {
+        double av[4], xv[4];
+        UNROLL for (int u = 0; u < 4; u++) { av[u] = a[e + 64 * u]; xv[u] = x[ci[e + 64 * u]] + xc[cagg[e + 64 * u]]; }
+        UNROLL for (int u = 0; u < 4; u++) r -= av[u] * xv[u];
+    }
+    for (; e < e1; e += 64) r -= a[e] * (x[ci[e]] + xc[cagg[e]]);
     xo[i] = (x[i] + xc[q >> 2]) + OMEGA * dinv[i] * r;
 }
 
@@ -169,7 +182,7 @@ __global__ void __launch_bounds__(256) amg_up(int64_t nq, const int64_t* __restr
 // inverse.  Launched level by level, those levels took four launches each and
 // a serial triangular solve (27 us), about 150 us of the cycle's 550 at
 // 500,000 rows; this kernel takes 25.
-constexpr int SM_ROWS = 3072, SM_TOP = 2048, SM_LEVELS = 14, SM_THREADS = 1024;
+constexpr int SM_ROWS = 1536, SM_TOP = 1024, SM_LEVELS = 14, SM_THREADS = 1024;
 struct SmallLevel {
     int n, nc, nq;
     const int64_t* off;
@@ -207,7 +220,14 @@ __global__ void __launch_bounds__(SM_THREADS) amg_small(SmallHier h, const doubl
             if (i >= 0) {
                 r = sb[o + i];
                 const int e1 = (int)L.off[(q >> 6) + 1];
-                for (int e = (int)L.off[q >> 6] + (q & 63); e < e1; e += 64) r -= L.a[e] * sx[o + L.ci[e]];
+                int e = (int)L.off[q >> 6] + (q & 63);
+                for (; e + 192 < e1; e += 256) {             // four entries in flight
+                    double av[4];
+                    int cv[4];
+                    UNROLL for (int u = 0; u < 4; u++) { av[u] = L.a[e + 64 * u]; cv[u] = L.ci[e + 64 * u]; }
+                    UNROLL for (int u = 0; u < 4; u++) r -= av[u] * sx[o + cv[u]];
+                }
+                for (; e < e1; e += 64) r -= L.a[e] * sx[o + L.ci[e]];
             }
             r += __shfl_xor(r, 1);
             r += __shfl_xor(r, 2);
@@ -238,8 +258,14 @@ __global__ void __launch_bounds__(SM_THREADS) amg_small(SmallHier h, const doubl
             if (i < 0) continue;
             double r = sb[o + i];
             const int e1 = (int)L.off[(q >> 6) + 1];
-            for (int e = (int)L.off[q >> 6] + (q & 63); e < e1; e += 64)
-                r -= L.a[e] * (sx[o + L.ci[e]] + sx[on + L.cagg[e]]);
+            int e = (int)L.off[q >> 6] + (q & 63);
+            for (; e + 192 < e1; e += 256) {
+                double av[4];
+                int cv[4], gv[4];
+                UNROLL for (int u = 0; u < 4; u++) { av[u] = L.a[e + 64 * u]; cv[u] = L.ci[e + 64 * u]; gv[u] = L.cagg[e + 64 * u]; }
+                UNROLL for (int u = 0; u < 4; u++) r -= av[u] * (sx[o + cv[u]] + sx[on + gv[u]]);
+            }
+            for (; e < e1; e += 64) r -= L.a[e] * (sx[o + L.ci[e]] + sx[on + L.cagg[e]]);
             so[i] = (sx[o + i] + sx[on + (q >> 2)]) + OMEGA * L.dinv[i] * r;
         }
         __syncthreads();
@@ -319,7 +345,7 @@ __global__ void __launch_bounds__(64) amg_dense_inv(int n, const double* __restr
 }
 
 // One colour of the block Gauss-Seidel sweep; a group of B lanes per row,
-// lane r = row r of the block.  The diagonal slot is first in each row.
+// lane r = column r of the blocks and row r of the result.  The diagonal slot is first in each row.
 template <int B>
 __global__ void __launch_bounds__(64) gs_color(const int32_t* __restrict__ rows, int64_t nrows,
                                                const int64_t* __restrict__ rowptr, const int32_t* __restrict__ col,
@@ -327,25 +353,19 @@ __global__ void __launch_bounds__(64) gs_color(const int32_t* __restrict__ rows,
                                                const double* __restrict__ rhat, double* __restrict__ x)
 {
     constexpr int G = 64 / B;
+    __shared__ double sh[64][B + 1];
     const int lane = threadIdx.x, g = lane / B, r = lane % B;
     const int64_t k = (int64_t)blockIdx.x * G + g;
     const bool valid = g < G && k < nrows;
     const int64_t i = valid ? rows[k] : 0;
-    double t = 0;
+    double acc[B];
+    UNROLL for (int c = 0; c < B; c++) acc[c] = 0;
     if (valid)
-        for (int64_t s = rowptr[i] + 1; s < rowptr[i + 1]; s++) {
-            const double* blk = val + ((size_t)s * B + r) * B;
-            const double* xm = x + (size_t)col[s] * B;
-            UNROLL for (int c = 0; c < B; c++) t += blk[c] * xm[c];
-        }
-    const int base = (g < G ? g : 0) * B;
-    double y = valid ? rhat[(size_t)i * B + r] : 0.0;
-    const double* d = dinv + ((size_t)i * B + r) * B;
-    UNROLL for (int c = 0; c < B; c++) {
-        const double tc = __shfl(t, base + c);
-        if (valid) y -= d[c] * tc;
-    }
-    if (valid) x[(size_t)i * B + r] = y;
+        for (int64_t s = rowptr[i] + 1; s < rowptr[i + 1]; s++) block_column<B>(val + (size_t)s * B * B, r, x[(size_t)col[s] * B + r], acc);
+    const double t = row_sums<B>(acc, sh);
+    UNROLL for (int c = 0; c < B; c++) acc[c] = dinv[((size_t)i * B + c) * B + r] * t;
+    const double y = row_sums<B>(acc, sh);
+    if (valid) x[(size_t)i * B + r] = rhat[(size_t)i * B + r] - y;
 }
 
 // R = v - Dinv J x1 and z = R + x1 on the bulk rows for the pressure
@@ -358,7 +378,7 @@ __global__ void __launch_bounds__(64) cpr_resid(const int64_t* __restrict__ rowp
 {
     constexpr int G = 64 / B;
     const int lane = threadIdx.x, g = lane / B, r = lane % B;
-    const int64_t i = (int64_t)blockIdx.x * G + g;
+    const int64_t i = xcd_chunk(blockIdx.x, gridDim.x) * G + g;
     if (g >= G || i >= nb) return;
     double t = 0;
     for (int64_t s = rowptr[i]; s < rowptr[i + 1]; s++) t += d0[(size_t)s * B + r] * px[col[s]];
@@ -375,7 +395,8 @@ __global__ void __launch_bounds__(64) cpr_resid(const int64_t* __restrict__ rowp
 // v2, and w1 = R1 + Dinv A12 g2 + v1 - R1 = v1 + Dinv A12 g2 (first colour).
 // R holds g afterwards.  One iteration reads the off-diagonal blocks once; the
 // sweep over both colours, the residual before it and the product after it read
-// the matrix three times (500,000 rows, B = 8: 0.47 + 0.36 + 0.36 ms, now 0.45).
+// the matrix three times (500,000 rows, B = 8: 0.47 + 0.36 + 0.36 ms, now 0.41, at
+// 4.8 TB/s the rate of a large copy).
 template <int B, bool SECOND>
 __global__ void __launch_bounds__(64) cpr_half(const int32_t* __restrict__ rows, int64_t nrows,
                                                const int64_t* __restrict__ rowptr, const int32_t* __restrict__ col,
@@ -384,53 +405,51 @@ __global__ void __launch_bounds__(64) cpr_half(const int32_t* __restrict__ rows,
                                                double* R, double* __restrict__ z, double* __restrict__ w)
 {
     constexpr int G = 64 / B;
+    __shared__ double sh[64][B + 1];
     const int lane = threadIdx.x, g = lane / B, r = lane % B;
-    const int64_t k = (int64_t)blockIdx.x * G + g;
+    const int64_t k = xcd_chunk(blockIdx.x, gridDim.x) * G + g;
     const bool valid = g < G && k < nrows;
     const int64_t i = valid ? rows[k] : 0;
-    double t = 0;
-    if (valid)
-        for (int64_t s = rowptr[i] + 1; s < rowptr[i + 1]; s++) {
-            const double* blk = val + ((size_t)s * B + r) * B;
-            const double* xm = R + (size_t)col[s] * B;
-            UNROLL for (int c = 0; c < B; c++) t += blk[c] * xm[c];
-        }
-    const int base = (g < G ? g : 0) * B;
-    const double* d = dinv + ((size_t)i * B + r) * B;
-    double y = 0;
-    UNROLL for (int c = 0; c < B; c++) {
-        const double tc = __shfl(t, base + c);
-        if (valid) y += d[c] * tc;
-    }
-    if (!valid) return;
     const size_t o = (size_t)i * B + r;
+    double d[B], acc[B];                           // column r of Dinv, loaded beside the blocks
+    UNROLL for (int c = 0; c < B; c++) { d[c] = dinv[((size_t)i * B + c) * B + r]; acc[c] = 0; }
+    const double vo = v[o];
+    if (valid)
+        for (int64_t s = rowptr[i] + 1; s < rowptr[i + 1]; s++) block_column<B>(val + (size_t)s * B * B, r, R[(size_t)col[s] * B + r], acc);
+    const double t = row_sums<B>(acc, sh);
+    UNROLL for (int c = 0; c < B; c++) acc[c] = d[c] * t;
+    const double y = row_sums<B>(acc, sh);
+    if (!valid) return;
     if constexpr (SECOND) {
         const double gi = R[o] - y;
         R[o] = gi;
         z[o] = r == 0 ? gi + px[i] : gi;
-        w[o] = v[o];
+        w[o] = vo;
     } else {
-        w[o] = v[o] + y;
+        w[o] = vo + y;
     }
 }
 
 // ------------------------------------------------- Gram-Schmidt of one vector
-// Classical Gram-Schmidt with one reorthogonalisation against M vectors in
-// three passes over them (h = V.w; w -= V h with h2 = V.w; w -= V h2 with w.w),
-// each element's M values held in registers, the partials summed by the last
-// block to finish.  Bandwidth-bound: a pass reads M + 1 vectors.  One pass per
-// product and per update, each reading w again for every vector, took 26 ms of
-// a 45-iteration solve of 4M unknowns; these take 14.
-constexpr int FG_THREADS = 256, FG_BLOCKS = 512, FG_MAX = 31;
+// Classical Gram-Schmidt with one reorthogonalisation against M vectors:
+// h = V.w; w -= V h with h2 = V.w; w -= V h2 with w.w.  Each block writes its
+// partial sums and a second kernel adds them in block order (letting the last
+// block to finish add them needs a device-wide release in every block, which
+// flushes the L2s: 130 us at 1,024 blocks).  Bandwidth-bound.  A thread takes E elements of a
+// contiguous tile and walks the vectors one after another, M accumulators in
+// registers: on 4M elements and M = 30, 6.4 TB/s for the product and 5.4 for
+// the update with E = 8, against 2.5 for a thread that loads its element of
+// all M vectors at once.  E = 1 for vectors that would leave the device idle.
+// Up to ORTH_M vectors the first update and the second product are one
+// kernel that reads the element's vectors again while they are near (M = 16:
+// 145 us against 99 + 89; M = 30: 358 against 182 + 154, so two above).
+constexpr int FG_THREADS = 256, FG_BLOCKS = 1024, FG_MAX = 31, FG_E = 8, ORTH_M = 16;
 
-// sums acc over the block into part, and returns true in the last block of
-// the grid, which then finds the M totals in tot (LDS, valid after the call)
+// the block's sums of acc into part[k][blockIdx.x] (FG_BLOCKS apart)
 template <int M>
-__device__ __forceinline__ bool fg_reduce(double (&acc)[M], double* part, unsigned* done, double* tot)
+__device__ __forceinline__ void fg_partial(double (&acc)[M], double* part)
 {
     __shared__ double sh[FG_THREADS / 64][32];
-    __shared__ double sums[8][32];
-    __shared__ bool last;
     const int t = threadIdx.x, wv = t >> 6, ln = t & 63;
     UNROLL for (int k = 0; k < M; k++) {
         double v = acc[k];
@@ -438,54 +457,118 @@ __device__ __forceinline__ bool fg_reduce(double (&acc)[M], double* part, unsign
         if (ln == 0) sh[wv][k] = v;
     }
     __syncthreads();
-    if (t < M) part[(size_t)blockIdx.x * 32 + t] = ((sh[0][t] + sh[1][t]) + sh[2][t]) + sh[3][t];
-    __threadfence();
-    __syncthreads();
-    if (t == 0) last = atomicAdd(done, 1u) == gridDim.x - 1;
-    __syncthreads();
-    if (!last) return false;
-    __threadfence();
-    const int k = t & 31, g = t >> 5;
-    double v = 0;
-    if (k < M)
-        for (unsigned b = g; b < gridDim.x; b += 8) v += __builtin_nontemporal_load(&part[(size_t)b * 32 + k]);
-    sums[g][k] = v;
-    __syncthreads();
-    if (t < M) {
-        double u = 0;
-        for (int q = 0; q < 8; q++) u += sums[q][t];
-        tot[t] = u;
-    }
-    if (t == 0) *done = 0;
-    __syncthreads();
-    return true;
+    if (t < M) part[(size_t)t * FG_BLOCKS + blockIdx.x] = ((sh[0][t] + sh[1][t]) + sh[2][t]) + sh[3][t];
 }
 
-template <int M>
-__global__ void __launch_bounds__(FG_THREADS) fg_dot(const double* __restrict__ V, int64_t ldv,
-                                                     const double* __restrict__ w, int64_t len, double* part,
-                                                     unsigned* done, double* __restrict__ h, double* host)
+// total of product blockIdx.x over the n blocks' partials: h (and host, when
+// given); with sum (one block) also host[k] = a[k] + b[k] for k < m, the total in
+// host[m] and its inverse root in scale
+__global__ void __launch_bounds__(FG_THREADS) fg_final(const double* __restrict__ part, int n, double* __restrict__ h,
+                                                       double* host, bool sum, int m, const double* __restrict__ a,
+                                                       const double* __restrict__ b, double* __restrict__ scale)
 {
-    __shared__ double tot[32];
+    __shared__ double sh[FG_THREADS];
+    const int t = threadIdx.x, k = blockIdx.x;
+    double v = 0;
+    UNROLL for (int q = 0; q < FG_BLOCKS / FG_THREADS; q++) {
+        const int i = q * FG_THREADS + t;
+        v += i < n ? part[(size_t)k * FG_BLOCKS + i] : 0.0;
+    }
+    sh[t] = v;
+    __syncthreads();
+    for (int o = FG_THREADS / 2; o > 0; o >>= 1) {
+        if (t < o) sh[t] += sh[t + o];
+        __syncthreads();
+    }
+    if (!sum) {
+        if (t == 0) {
+            h[k] = sh[0];
+            if (host) host[k] = sh[0];
+        }
+        return;
+    }
+    if (t < m) host[t] = a[t] + b[t];
+    if (t == 0) {
+        host[m] = sh[0];
+        *scale = 1 / sqrt(sh[0]);
+    }
+}
+
+// E elements of p at i + 256 e; FULL: the block's whole tile lies below len,
+// else 0 past the end
+template <int E, bool FULL>
+__device__ __forceinline__ void fg_load(const double* __restrict__ p, int64_t i, int64_t len, double (&v)[E])
+{
+    UNROLL for (int e = 0; e < E; e++) v[e] = FULL || i + FG_THREADS * e < len ? p[i + FG_THREADS * e] : 0.0;
+}
+
+template <int M, int E, bool FULL>
+__device__ __forceinline__ void fg_dot_tile(const double* __restrict__ V, int64_t ldv, const double* __restrict__ w,
+                                            int64_t i, int64_t len, double (&acc)[M])
+{
+    double wi[E];
+    fg_load<E, FULL>(w, i, len, wi);
+    UNROLL for (int k = 0; k < M; k++) {
+        double v[E];
+        fg_load<E, FULL>(V + (size_t)k * ldv, i, len, v);
+        UNROLL for (int e = 0; e < E; e++) acc[k] += v[e] * wi[e];
+    }
+}
+
+template <int M, int E>
+__global__ void __launch_bounds__(FG_THREADS) fg_dot(const double* __restrict__ V, int64_t ldv,
+                                                     const double* __restrict__ w, int64_t len, double* part)
+{
+    constexpr int64_t TILE = (int64_t)FG_THREADS * E;
     double acc[M];
     UNROLL for (int k = 0; k < M; k++) acc[k] = 0;
-    for (int64_t i = (int64_t)blockIdx.x * FG_THREADS + threadIdx.x; i < len; i += (int64_t)gridDim.x * FG_THREADS) {
-        const double wi = w[i];
-        UNROLL for (int k = 0; k < M; k++) acc[k] += V[(size_t)k * ldv + i] * wi;
+    int64_t b = (int64_t)blockIdx.x * TILE;
+    for (; b + TILE <= len; b += gridDim.x * TILE) fg_dot_tile<M, E, true>(V, ldv, w, b + threadIdx.x, len, acc);
+    if (b < len) fg_dot_tile<M, E, false>(V, ldv, w, b + threadIdx.x, len, acc);
+    fg_partial<M>(acc, part);
+}
+
+template <int M, int E, bool FULL>
+__device__ __forceinline__ void fg_update_tile(double* __restrict__ w, const double* __restrict__ V, int64_t ldv,
+                                               const double* cs, int64_t i, int64_t len, double& nn)
+{
+    double wi[E];
+    fg_load<E, FULL>(w, i, len, wi);
+    UNROLL for (int k = 0; k < M; k++) {
+        double v[E];
+        fg_load<E, FULL>(V + (size_t)k * ldv, i, len, v);
+        UNROLL for (int e = 0; e < E; e++) wi[e] -= cs[k] * v[e];
     }
-    if (!fg_reduce<M>(acc, part, done, tot)) return;
-    if (threadIdx.x < M) {
-        h[threadIdx.x] = tot[threadIdx.x];
-        if (host) host[threadIdx.x] = tot[threadIdx.x];
+    UNROLL for (int e = 0; e < E; e++) {
+        if (FULL || i + FG_THREADS * e < len) w[i + FG_THREADS * e] = wi[e];
+        nn += wi[e] * wi[e];
     }
+}
+
+// w -= V c; with NORM, also the partials of w.w
+template <int M, int E, bool NORM>
+__global__ void __launch_bounds__(FG_THREADS) fg_update(double* __restrict__ w, const double* __restrict__ V,
+                                                        int64_t ldv, const double* __restrict__ c, int64_t len,
+                                                        double* part)
+{
+    constexpr int64_t TILE = (int64_t)FG_THREADS * E;
+    __shared__ double cs[32];
+    if (threadIdx.x < M) cs[threadIdx.x] = c[threadIdx.x];
+    __syncthreads();
+    double acc[1] = {0};
+    int64_t b = (int64_t)blockIdx.x * TILE;
+    for (; b + TILE <= len; b += gridDim.x * TILE)
+        fg_update_tile<M, E, true>(w, V, ldv, cs, b + threadIdx.x, len, acc[0]);
+    if (b < len) fg_update_tile<M, E, false>(w, V, ldv, cs, b + threadIdx.x, len, acc[0]);
+    if constexpr (NORM) fg_partial<1>(acc, part);
 }
 
 template <int M>
 __global__ void __launch_bounds__(FG_THREADS) fg_orth(double* __restrict__ w, const double* __restrict__ V,
                                                       int64_t ldv, const double* __restrict__ h, int64_t len,
-                                                      double* part, unsigned* done, double* __restrict__ h2)
+                                                      double* part)
 {
-    __shared__ double tot[32], hs[32];
+    __shared__ double hs[32];
     if (threadIdx.x < M) hs[threadIdx.x] = h[threadIdx.x];
     __syncthreads();
     double acc[M];
@@ -498,35 +581,7 @@ __global__ void __launch_bounds__(FG_THREADS) fg_orth(double* __restrict__ w, co
         w[i] = wi;
         UNROLL for (int k = 0; k < M; k++) acc[k] += v[k] * wi;
     }
-    if (!fg_reduce<M>(acc, part, done, tot)) return;
-    if (threadIdx.x < M) h2[threadIdx.x] = tot[threadIdx.x];
-}
-
-template <int M>
-__global__ void __launch_bounds__(FG_THREADS) fg_orth_norm(double* __restrict__ w, const double* __restrict__ V,
-                                                           int64_t ldv, const double* __restrict__ h,
-                                                           const double* __restrict__ h2, int64_t len, double* part,
-                                                           unsigned* done, double* host, double* __restrict__ scale)
-{
-    __shared__ double tot[32], hs[32];
-    const int t = threadIdx.x;
-    if (t < M) hs[t] = h2[t];
-    __syncthreads();
-    double acc[1] = {0};
-    for (int64_t i = (int64_t)blockIdx.x * FG_THREADS + t; i < len; i += (int64_t)gridDim.x * FG_THREADS) {
-        double v[M];
-        UNROLL for (int k = 0; k < M; k++) v[k] = V[(size_t)k * ldv + i];
-        double wi = w[i];
-        UNROLL for (int k = 0; k < M; k++) wi -= hs[k] * v[k];
-        w[i] = wi;
-        acc[0] += wi * wi;
-    }
-    if (!fg_reduce<1>(acc, part, done, tot)) return;
-    if (t < M) host[t] = h[t] + hs[t];
-    if (t == 0) {
-        host[M] = tot[0];
-        *scale = 1 / sqrt(tot[0]);
-    }
+    fg_partial<M>(acc, part);
 }
 
 template <int B>
@@ -760,47 +815,73 @@ hipError_t run_fg_scale(int B, double* v, const double* w, const double* scale, 
 
 int fg_scratch_len() { return FG_BLOCKS * 32; }
 
-static unsigned fg_blocks(int64_t len)
+// blocks of tiles of e elements per thread, and whether E = 8 fills the device
+static unsigned fg_blocks(int64_t len, int e)
 {
-    const int64_t b = (len + FG_THREADS - 1) / FG_THREADS;
+    const int64_t b = (len + (int64_t)FG_THREADS * e - 1) / ((int64_t)FG_THREADS * e);
     return (unsigned)(b < 1 ? 1 : (b > FG_BLOCKS ? FG_BLOCKS : b));
 }
+static bool fg_wide(int64_t len) { return len >= (int64_t)512 * FG_THREADS * FG_E; }
 
-#define OCPX_M_SWITCH(X)                                                                            \
-    switch (m) {                                                                                    \
-    X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17)    \
-    X(18) X(19) X(20) X(21) X(22) X(23) X(24) X(25) X(26) X(27) X(28) X(29) X(30) X(31)             \
-    default: return hipErrorInvalidValue;                                                           \
-    }
+#define OCPX_M_LOW(X) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16)
+#define OCPX_M_HIGH(X) X(17) X(18) X(19) X(20) X(21) X(22) X(23) X(24) X(25) X(26) X(27) X(28) X(29) X(30) X(31)
+static_assert(FG_MAX == 31 && ORTH_M == 16, "the cases of OCPX_M_LOW and OCPX_M_HIGH");
 
-hipError_t run_fg_dot(const double* V, int64_t ldv, int m, const double* w, int64_t len, double* part, unsigned* done,
-                      double* h, double* host, hipStream_t st)
+static hipError_t fg_sum(const double* part, unsigned n, int m, double* h, double* host, hipStream_t st)
 {
-    static_assert(FG_MAX == 31, "the cases of OCPX_M_SWITCH");
-#define X(M) case M: hipLaunchKernelGGL(fg_dot<M>, dim3(fg_blocks(len)), dim3(FG_THREADS), 0, st, V, ldv, w, len, part, done, h, host); break;
-    OCPX_M_SWITCH(X)
-#undef X
+    hipLaunchKernelGGL(fg_final, dim3(m), dim3(FG_THREADS), 0, st, part, (int)n, h, host, false, 0, nullptr, nullptr, nullptr);
     return hipGetLastError();
+}
+
+hipError_t run_fg_dot(const double* V, int64_t ldv, int m, const double* w, int64_t len, double* part, double* h,
+                      double* host, hipStream_t st)
+{
+    const unsigned nw = fg_blocks(len, FG_E), n1 = fg_blocks(len, 1);
+#define X(M) case M: if (fg_wide(len)) hipLaunchKernelGGL((fg_dot<M, FG_E>), dim3(nw), dim3(FG_THREADS), 0, st, V, ldv, w, len, part); \
+        else hipLaunchKernelGGL((fg_dot<M, 1>), dim3(n1), dim3(FG_THREADS), 0, st, V, ldv, w, len, part); break;
+    switch (m) {
+    OCPX_M_LOW(X) OCPX_M_HIGH(X)
+    default: return hipErrorInvalidValue;
+    }
+#undef X
+    return fg_sum(part, fg_wide(len) ? nw : n1, m, h, host, st);
 }
 
 hipError_t run_fg_orth(double* w, const double* V, int64_t ldv, int m, const double* h, int64_t len, double* part,
-                       unsigned* done, double* h2, hipStream_t st)
+                       double* h2, hipStream_t st)
 {
-#define X(M) case M: hipLaunchKernelGGL(fg_orth<M>, dim3(fg_blocks(len)), dim3(FG_THREADS), 0, st, w, V, ldv, h, len, part, done, h2); break;
-    OCPX_M_SWITCH(X)
+    const unsigned nw = fg_blocks(len, FG_E), n1 = fg_blocks(len, 1);
+#define X(M) case M: hipLaunchKernelGGL(fg_orth<M>, dim3(n1), dim3(FG_THREADS), 0, st, w, V, ldv, h, len, part); \
+        return fg_sum(part, n1, m, h2, nullptr, st);
+#define Y(M) case M: if (fg_wide(len)) hipLaunchKernelGGL((fg_update<M, FG_E, false>), dim3(nw), dim3(FG_THREADS), 0, st, w, V, ldv, h, len, part); \
+        else hipLaunchKernelGGL((fg_update<M, 1, false>), dim3(n1), dim3(FG_THREADS), 0, st, w, V, ldv, h, len, part); break;
+    switch (m) {
+    OCPX_M_LOW(X) OCPX_M_HIGH(Y)
+    default: return hipErrorInvalidValue;
+    }
 #undef X
-    return hipGetLastError();
+#undef Y
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? run_fg_dot(V, ldv, m, w, len, part, h2, nullptr, st) : e;
 }
 
 hipError_t run_fg_orth_norm(double* w, const double* V, int64_t ldv, int m, const double* h, const double* h2,
-                            int64_t len, double* part, unsigned* done, double* host, double* scale, hipStream_t st)
+                            int64_t len, double* part, double* host, double* scale, hipStream_t st)
 {
-#define X(M) case M: hipLaunchKernelGGL(fg_orth_norm<M>, dim3(fg_blocks(len)), dim3(FG_THREADS), 0, st, w, V, ldv, h, h2, len, part, done, host, scale); break;
-    OCPX_M_SWITCH(X)
+    const unsigned nw = fg_blocks(len, FG_E), n1 = fg_blocks(len, 1);
+#define X(M) case M: if (fg_wide(len)) hipLaunchKernelGGL((fg_update<M, FG_E, true>), dim3(nw), dim3(FG_THREADS), 0, st, w, V, ldv, h2, len, part); \
+        else hipLaunchKernelGGL((fg_update<M, 1, true>), dim3(n1), dim3(FG_THREADS), 0, st, w, V, ldv, h2, len, part); break;
+    switch (m) {
+    OCPX_M_LOW(X) OCPX_M_HIGH(X)
+    default: return hipErrorInvalidValue;
+    }
 #undef X
+    hipLaunchKernelGGL(fg_final, dim3(1), dim3(FG_THREADS), 0, st, part, (int)(fg_wide(len) ? nw : n1), nullptr, host, true, m, h,
+                       h2, scale);
     return hipGetLastError();
 }
-#undef OCPX_M_SWITCH
+#undef OCPX_M_LOW
+#undef OCPX_M_HIGH
 
 hipError_t run_fg_axpy(double* x, const double* Z, int64_t ldz, int m, const FgCoef& y, int64_t len, hipStream_t st)
 {

@@ -91,20 +91,19 @@ private:
 hipError_t run_gs_color(int B, const int32_t* rows, int64_t nrows, const int64_t* rowptr, const int32_t* col,
                         const double* val, const double* dinv, const double* rhat, double* x, hipStream_t st);
 
-// ---- FGMRES pieces on vectors of len doubles (the last block of each
-// reduction sums the partials in block order, so results have the same bits on
-// every run).  part: fg_scratch_len() doubles; done: one word, 0 before the
-// first call and after every call.
+// ---- FGMRES pieces on vectors of len doubles (partials are summed in block
+// order, so results have the same bits on every run).  part: fg_scratch_len()
+// doubles.
 int fg_scratch_len();
 // h[k] = V_k . w for k < m (V: m vectors, stride ldv; m <= 31); host (pinned, may be null) gets a copy
-hipError_t run_fg_dot(const double* V, int64_t ldv, int m, const double* w, int64_t len, double* part, unsigned* done,
-                      double* h, double* host, hipStream_t st);
+hipError_t run_fg_dot(const double* V, int64_t ldv, int m, const double* w, int64_t len, double* part, double* h,
+                      double* host, hipStream_t st);
 // w -= sum h[k] V_k, then h2[k] = V_k . w
 hipError_t run_fg_orth(double* w, const double* V, int64_t ldv, int m, const double* h, int64_t len, double* part,
-                       unsigned* done, double* h2, hipStream_t st);
+                       double* h2, hipStream_t st);
 // w -= sum h2[k] V_k; host[k] = h[k] + h2[k], host[m] = w . w; *scale = 1 / |w|
 hipError_t run_fg_orth_norm(double* w, const double* V, int64_t ldv, int m, const double* h, const double* h2,
-                            int64_t len, double* part, unsigned* done, double* host, double* scale, hipStream_t st);
+                            int64_t len, double* part, double* host, double* scale, hipStream_t st);
 // v = w * (scale ? *scale : s); for the nb bulk rows pb = v's pressure entries and px0 = OMEGA dinv0 pb
 hipError_t run_fg_scale(int B, double* v, const double* w, const double* scale, double s, int64_t nb, int64_t len,
                         const double* dinv0, double* pb, double* px0, hipStream_t st);

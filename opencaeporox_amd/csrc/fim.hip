@@ -158,16 +158,6 @@ __global__ void __launch_bounds__(64) krpc_aux(const DevSat* __restrict__ sp, co
     }
 }
 
-// Blocks are dealt to the 8 XCDs round-robin (block b runs on XCD b % 8).
-// Renumber them so each XCD works through one contiguous chunk of rows and
-// the neighbour records a row reads stay in that XCD's L2.
-__device__ __forceinline__ int64_t xcd_chunk(int64_t b, int64_t nblk)
-{
-    constexpr int64_t X = 8;
-    const int64_t x = b % X, k = b / X, q = nblk / X, r = nblk % X;
-    return x * q + (x < r ? x : r) + k;
-}
-
 // --------------------------------------------------------- residual + Jacobian
 // Upwinding of one phase (OCPConvection01::CalFlux :37-78).  Returns false
 // when the phase carries no flux.

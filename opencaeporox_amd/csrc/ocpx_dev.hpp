@@ -63,6 +63,16 @@ __device__ __forceinline__ int items_per_wave(unsigned total, int per)
     return l < 1u ? 1 : (l > (unsigned)per ? per : (int)l);
 }
 
+// Blocks are dealt to the 8 XCDs round-robin (block b runs on XCD b % 8).
+// Renumber them so each XCD works through one contiguous chunk of rows and
+// the neighbour records a row reads stay in that XCD's L2.
+__device__ __forceinline__ int64_t xcd_chunk(int64_t b, int64_t nblk)
+{
+    constexpr int64_t X = 8;
+    const int64_t x = b % X, k = b / X, q = nblk / X, r = nblk % X;
+    return x * q + (x < r ? x : r) + k;
+}
+
 // finite test usable on host and device (v - v is NaN for inf and NaN)
 OCPX_HD bool finite_d(double v) { return (v - v) == 0.0; }
 

@@ -127,7 +127,6 @@ struct ocpx_ctx {
     double *fg_V = nullptr, *fg_Z = nullptr, *fg_w = nullptr, *fg_t = nullptr, *fg_x1 = nullptr;
     double *fg_r2 = nullptr, *fg_px = nullptr, *fg_h = nullptr, *fg_part = nullptr;
     double* fg_d0 = nullptr;             // [nnzb][b] column 0 of every decoupled block
-    unsigned* fg_done = nullptr;         // blocks of the current reduction that are done
     double* fg_host = nullptr;           // pinned: the Hessenberg column and the norm of each iteration
     int64_t fg_cap = 0;
     // timing
@@ -1427,8 +1426,7 @@ int fgmres_cpr(ocpx_ctx* c, const double* rhs, int64_t len, int32_t nwj, double 
     }
     if (!c->fg_host) {
         if ((rc = dalloc(c, &c->fg_px, (size_t)nb)) || (rc = dalloc(c, &c->fg_d0, (size_t)c->nnzb * B)) ||
-            (rc = dalloc(c, &c->fg_h, 128)) || (rc = dalloc(c, &c->fg_part, (size_t)fg_scratch_len())) ||
-            (rc = dalloc(c, &c->fg_done, 1)))
+            (rc = dalloc(c, &c->fg_h, 128)) || (rc = dalloc(c, &c->fg_part, (size_t)fg_scratch_len())))
             return rc;
         HIPCHK(c, hipHostMalloc((void**)&c->fg_host, 64 * sizeof(double), hipHostMallocDefault));
     }
@@ -1479,7 +1477,7 @@ int fgmres_cpr(ocpx_ctx* c, const double* rhs, int64_t len, int32_t nwj, double 
     if (nwj) HIPCHK(c, run_bsr_spmv(B, nullptr, nullptr, c->dinv_w, rhs + nb * B, w + nb * B, nwj, st));
     HIPCHK(c, run_axpbypcz(x, nullptr, 0, nullptr, 0, nullptr, len, st));
     auto norm_w = [&](double& out) -> int {
-        HIPCHK(c, run_fg_dot(w, len, 1, w, len, c->fg_part, c->fg_done, dh, c->fg_host, st));
+        HIPCHK(c, run_fg_dot(w, len, 1, w, len, c->fg_part, dh, c->fg_host, st));
         HIPCHK(c, hipStreamSynchronize(st));
         out = std::sqrt(host[0]);
         return OCPX_OK;
@@ -1503,9 +1501,9 @@ int fgmres_cpr(ocpx_ctx* c, const double* rhs, int64_t len, int32_t nwj, double 
             HIPCHK(c, run_fg_scale(B, Vj, w, j ? dscale : nullptr, 1.0 / beta, nb, len, amg.level0_dinv(), amg.level0_b(),
                                    amg.level0_x(), st));
             if ((rc = precond_op(Vj, Zj))) return rc;
-            HIPCHK(c, run_fg_dot(V, len, j + 1, w, len, c->fg_part, c->fg_done, dh, nullptr, st));
-            HIPCHK(c, run_fg_orth(w, V, len, j + 1, dh, len, c->fg_part, c->fg_done, dh2, st));
-            HIPCHK(c, run_fg_orth_norm(w, V, len, j + 1, dh, dh2, len, c->fg_part, c->fg_done, c->fg_host, dscale, st));
+            HIPCHK(c, run_fg_dot(V, len, j + 1, w, len, c->fg_part, dh, nullptr, st));
+            HIPCHK(c, run_fg_orth(w, V, len, j + 1, dh, len, c->fg_part, dh2, st));
+            HIPCHK(c, run_fg_orth_norm(w, V, len, j + 1, dh, dh2, len, c->fg_part, c->fg_host, dscale, st));
             HIPCHK(c, hipStreamSynchronize(st));
             const double hn = std::sqrt(host[j + 1]);
             for (int i = 0; i <= j; i++) H[i * M + j] = host[i];

@@ -245,6 +245,32 @@ hipError_t run_well_bhp_update(ocpx_well* wells, int32_t nwell, int B, int64_t n
 hipError_t run_get_solution(int nc, double* P, double* Ni, double* S, double* xij,
                             const double* dXsdXp, const double* u, double dSmax, int64_t nb,
                             hipStream_t st);
+// Block rows times vectors, a group of B lanes per row: lane r takes column r
+// of every block, so each load of the group is one contiguous row of B doubles
+// (a lane per block row read its 8 B bytes in pieces B apart, eight lines per
+// instruction instead of one), keeps one partial per row in acc, and the
+// partials cross the lanes once per block row through LDS.
+template <int B>
+__device__ __forceinline__ void block_column(const double* __restrict__ blk, int r, double x, double (&acc)[B])
+{
+#pragma unroll
+    for (int c = 0; c < B; c++) acc[c] += blk[c * B + r] * x;
+}
+// sum over the group's lanes of their acc[r] for lane r; one-wavefront blocks
+template <int B>
+__device__ __forceinline__ double row_sums(const double (&acc)[B], double (*sh)[B + 1])
+{
+    const int lane = threadIdx.x, g = lane / B, r = lane % B, base = (g < 64 / B ? g : 0) * B;
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < B; c++) sh[lane][c] = acc[c];
+    __syncthreads();
+    double t = 0;
+#pragma unroll
+    for (int c = 0; c < B; c++) t += sh[base + c][r];
+    return t;
+}
+
 // linear solve (solver.hip)
 hipError_t run_bsr_diag_inv(int B, const int64_t* rowptr, const double* val, int64_t nb, double* dinv,
                             hipStream_t st);

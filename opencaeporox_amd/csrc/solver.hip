@@ -12,9 +12,8 @@
 //    block and of the identity; Gauss-Jordan with partial pivoting, the
 //    pivot column broadcast from its lane.
 //  - bsr_spmv (also the block-diagonal apply): one block row per b lanes,
-//    lane r = row r; a lane reads row r of each block (b contiguous
-//    doubles, the b lanes of a row read b*b contiguous doubles) and the b
-//    entries of x it multiplies.
+//    lane r = column r of each block and entry r of x; the lanes' partial
+//    sums are exchanged once per row.
 //  - dot: fixed-shape block partial sums, then one block sums them in
 //    order, so a dot product has the same bits on every run.
 #include "ocpx_dev.hpp"
@@ -74,18 +73,19 @@ __global__ void __launch_bounds__(64) bsr_spmv(const int64_t* __restrict__ rowpt
                                                double* __restrict__ y, int64_t nb)
 {
     constexpr int G = 64 / B;
+    __shared__ double sh[64][B + 1];
     const int lane = threadIdx.x, g = lane / B, r = lane % B;
     const int64_t n = (int64_t)blockIdx.x * G + g;
-    if (g >= G || n >= nb) return;
-    const int64_t s0 = rowptr ? rowptr[n] : n, s1 = rowptr ? rowptr[n + 1] : n + 1;
-    double acc = 0;
+    const bool valid = g < G && n < nb;
+    const int64_t s0 = !valid ? 0 : (rowptr ? rowptr[n] : n), s1 = !valid ? 0 : (rowptr ? rowptr[n + 1] : n + 1);
+    double acc[B];
+    UNROLL for (int c = 0; c < B; c++) acc[c] = 0;
     for (int64_t s = s0; s < s1; s++) {
         const int64_t m = rowptr ? (int64_t)col[s] : n;
-        const double* blk = val + ((size_t)s * B + r) * B;
-        const double* xm = x + (size_t)m * B;
-        UNROLL for (int c = 0; c < B; c++) acc += blk[c] * xm[c];
+        block_column<B>(val + (size_t)s * B * B, r, x[(size_t)m * B + r], acc);
     }
-    y[(size_t)n * B + r] = acc;
+    const double t = row_sums<B>(acc, sh);
+    if (valid) y[(size_t)n * B + r] = t;
 }
 
 constexpr int DOT_BLOCKS = 1024, DOT_THREADS = 256;
