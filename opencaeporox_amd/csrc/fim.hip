@@ -94,6 +94,7 @@ __global__ void __launch_bounds__(64) krpc_aux(const DevSat* __restrict__ sp, co
 {
     constexpr int nc = NCB, B = nc + 1, np = 3, G = 64 / B, REC = np * B * B, RL = aux_len(B, nc);
     constexpr int SV = 24, SX = 24 + 9 * B;
+    __shared__ double dsh[G][3][nc];
     const int lane = threadIdx.x, g = lane / B, r = lane % B;
     const int64_t n = (int64_t)blockIdx.x * G + g;
     if (g >= G || n >= c.nb) return;
@@ -124,20 +125,35 @@ __global__ void __launch_bounds__(64) krpc_aux(const DevSat* __restrict__ sp, co
     double* A = c.aux + (size_t)n * RL;
     const double one = r == 0 ? 1.0 : 0.0;
     const double depth = c.depth[n];
+    const unsigned long long group = ((1ull << B) - 1ull) << (g * B);
     UNROLL for (int j = 0; j < np; j++) {
         const bool ex = c.phaseExist[j * nb + n] != 0;
         double drho = 0, dxi = 0, dmu = 0;
+        bool hasx = false;                    // the phase's composition depends on the primary variables
         if (ex) {
             drho = one * c.rhoP[j * nb + n];
             dxi = one * c.xiP[j * nb + n];
             dmu = one * c.muP[j * nb + n];
-            UNROLL for (int m = 0; m < nc; m++) {
-                const double xm = X[(np + j * nc + m) * B + r];
-                drho += c.rhox[(size_t)(j * nc + m) * nb + n] * xm;
-                dxi += c.xix[(size_t)(j * nc + m) * nb + n] * xm;
-                dmu += c.mux[(size_t)(j * nc + m) * nb + n] * xm;
+            // lane m loads component m's derivatives for the cell's lanes
+            // (each lane all of them: 0.75 ms at 100x100x50, b = 8; so 0.63)
+            if (r < nc) {
+                dsh[g][0][r] = c.rhox[(size_t)(j * nc + r) * nb + n];
+                dsh[g][1][r] = c.xix[(size_t)(j * nc + r) * nb + n];
+                dsh[g][2][r] = c.mux[(size_t)(j * nc + r) * nb + n];
             }
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // one wavefront: its LDS operations run in order
+        if (ex) {
+            UNROLL for (int m = 0; m < nc; m++) {
+                const double xm = X[(np + j * nc + m) * B + r];
+                hasx = hasx || xm != 0;
+                drho += dsh[g][0][m] * xm;
+                dxi += dsh[g][1][m] * xm;
+                dmu += dsh[g][2][m] * xm;
+            }
+        }
+        const bool anyx = (__ballot(hasx) & group) != 0;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         double dkr = 0, dPj = one;
         UNROLL for (int k = 0; k < np; k++) { dkr += dk[j * 3 + k] * dS[k]; dPj += dp[j * 3 + k] * dS[k]; }
         const double xi = c.xi[j * nb + n], mu = c.mu[j * nb + n];
@@ -152,7 +168,7 @@ __global__ void __launch_bounds__(64) krpc_aux(const DevSat* __restrict__ sp, co
         if (r < nc) A[SX + j * nc + r] = c.xij[(size_t)(j * nc + r) * nb + n];
         if (r < 4) {                          // the phase's 8 scalars, one 16-byte pair per lane
             const double v0 = r == 0 ? c.rho[j * nb + n] : (r == 1 ? xi : (r == 2 ? mu : lam));
-            const double v1 = r == 0 ? P + pc[j] : (r == 1 ? kr[j] : (r == 2 ? (ex ? 1.0 : 0.0) : depth));
+            const double v1 = r == 0 ? P + pc[j] : (r == 1 ? kr[j] : (r == 2 ? (ex ? (anyx ? 2.0 : 1.0) : 0.0) : depth));
             reinterpret_cast<double2*>(A + 8 * j)[r] = make_double2(v0, v1);
         }
     }
@@ -185,23 +201,16 @@ OCPX_HD bool upwind(const CellIO& c, size_t nb, int64_t b, int64_t e, int j, Upw
 // bmax/barg[2 * block + {0, 1}].
 __device__ __forceinline__ void block_norms(double absV, double absN, int64_t idx, double* bmax, int64_t* barg)
 {
-    __shared__ double sV[64], sN[64];
-    __shared__ int64_t iV[64], iN[64];
-    const int lane = threadIdx.x;
-    sV[lane] = absV; iV[lane] = idx;
-    sN[lane] = absN; iN[lane] = idx;
-    __syncthreads();
-    for (int w = 32; w > 0; w >>= 1) {
-        if (lane < w) {
-            const int o = lane + w;
-            if (sV[o] > sV[lane] || (sV[o] == sV[lane] && iV[o] < iV[lane])) { sV[lane] = sV[o]; iV[lane] = iV[o]; }
-            if (sN[o] > sN[lane] || (sN[o] == sN[lane] && iN[o] < iN[lane])) { sN[lane] = sN[o]; iN[lane] = iN[o]; }
-        }
-        __syncthreads();
+    int iv = idx > INT32_MAX ? INT32_MAX : (int)idx, in = iv;         // cells fit 32 bits
+    for (int o = 32; o > 0; o >>= 1) {
+        const double v2 = __shfl_xor(absV, o), n2 = __shfl_xor(absN, o);
+        const int i2 = __shfl_xor(iv, o), j2 = __shfl_xor(in, o);
+        if (v2 > absV || (v2 == absV && i2 < iv)) { absV = v2; iv = i2; }
+        if (n2 > absN || (n2 == absN && j2 < in)) { absN = n2; in = j2; }
     }
-    if (lane == 0) {
-        bmax[2 * blockIdx.x] = sV[0]; barg[2 * blockIdx.x] = iV[0];
-        bmax[2 * blockIdx.x + 1] = sN[0]; barg[2 * blockIdx.x + 1] = iN[0];
+    if (threadIdx.x == 0) {
+        bmax[2 * blockIdx.x] = absV; barg[2 * blockIdx.x] = iv;
+        bmax[2 * blockIdx.x + 1] = absN; barg[2 * blockIdx.x + 1] = in;
     }
 }
 
@@ -368,10 +377,15 @@ __global__ void __launch_bounds__(64) res_asm(CellIO c, ConnIO cn, BsrIO bsr, do
                 const double ve = -Ve[B + r] - dGamma * (we * Ve[2 * B + r]);
                 const double dl = (upIsB ? Vb : Ve)[r];
                 const double Tdp = T * dP;
+                // dx_ij/dX of the upstream cell, read only where krpc_aux saw an
+                // entry that is not zero (never for water); 100x100x50, b = 8: 1.36 -> 1.28 ms
                 const double* XU = c.dXsdXp + (size_t)U * REC + (size_t)(np + j * nc) * B + r;
+                double dx[nc];
+                if (LU[8 * j + 5] > 1) UNROLL for (int i = 0; i < nc; i++) dx[i] = XU[i * B];
+                else UNROLL for (int i = 0; i < nc; i++) dx[i] = 0;
                 UNROLL for (int i = 0; i < nc; i++) {
                     const double tIJ = x[i] * xi * tJ;
-                    const double up = Tdp * (x[i] * dl + lam * XU[i * B]);
+                    const double up = Tdp * (x[i] * dl + lam * dx[i]);
                     rb[i] += tIJ * vb + (upIsB ? up : 0.0);
                     re[i] += tIJ * ve + (upIsB ? 0.0 : up);
                 }
@@ -402,6 +416,40 @@ __global__ void __launch_bounds__(64) res_asm(CellIO c, ConnIO cn, BsrIO bsr, do
         if (r > 0) absN = fabs(res / c.Nt[n]);
     }
     block_norms(absV, absN, valid ? n : INT64_MAX, bmax, barg);
+}
+
+// the per-block maxima down to one pair per block of this grid (NF_BLOCKS):
+// one block walking the 62,500 pairs of a 500,000-cell grid at B = 8 took 134 us,
+// the two launches take 10
+constexpr int NF_BLOCKS = 128;
+__global__ void __launch_bounds__(256) norms_part(int64_t nblk, const double* __restrict__ bmax,
+                                                  const int64_t* __restrict__ barg, double* __restrict__ pmax,
+                                                  int64_t* __restrict__ parg)
+{
+    __shared__ double sv[256], sn[256];
+    __shared__ int64_t iv[256], in_[256];
+    const int t = threadIdx.x;
+    double v = -1, w = -1;
+    int64_t a = INT64_MAX, b = INT64_MAX;
+    for (int64_t k = (int64_t)blockIdx.x * 256 + t; k < nblk; k += NF_BLOCKS * 256) {
+        const double v2 = bmax[2 * k], w2 = bmax[2 * k + 1];
+        const int64_t a2 = barg[2 * k], b2 = barg[2 * k + 1];
+        if (v2 > v || (v2 == v && a2 < a)) { v = v2; a = a2; }
+        if (w2 > w || (w2 == w && b2 < b)) { w = w2; b = b2; }
+    }
+    sv[t] = v; iv[t] = a; sn[t] = w; in_[t] = b;
+    __syncthreads();
+    for (int s = 128; s > 0; s >>= 1) {
+        if (t < s) {
+            if (sv[t + s] > sv[t] || (sv[t + s] == sv[t] && iv[t + s] < iv[t])) { sv[t] = sv[t + s]; iv[t] = iv[t + s]; }
+            if (sn[t + s] > sn[t] || (sn[t + s] == sn[t] && in_[t + s] < in_[t])) { sn[t] = sn[t + s]; in_[t] = in_[t + s]; }
+        }
+        __syncthreads();
+    }
+    if (t == 0) {
+        pmax[2 * blockIdx.x] = sv[0]; parg[2 * blockIdx.x] = iv[0];
+        pmax[2 * blockIdx.x + 1] = sn[0]; parg[2 * blockIdx.x + 1] = in_[0];
+    }
 }
 
 __global__ void __launch_bounds__(256) norms_final(int64_t nblk, const double* __restrict__ bmax,
@@ -602,9 +650,21 @@ hipError_t run_res_norms(int nc, const CellIO& c, const double* res, double* bma
 #undef X
 }
 
-hipError_t run_norms_final(int64_t nblocks, const double* bmax, const int64_t* barg, double* out4, hipStream_t st)
+int norms_scratch_len() { return 2 * NF_BLOCKS; }
+
+// the pairs of the residual kernels' blocks to norms4; above 1,024 blocks (where the
+// one block's walk, 2 us per 1,000, passes the second launch's 5 us) through one
+// pair per block of norms_part, kept behind them (norms_scratch_len() entries)
+hipError_t run_norms_final(int64_t nblocks, double* bmax, int64_t* barg, double* out4, hipStream_t st)
 {
-    hipLaunchKernelGGL(norms_final, dim3(1), dim3(256), 0, st, nblocks, bmax, barg, out4);
+    if (nblocks > 1024) {
+        double* pmax = bmax + 2 * nblocks;
+        int64_t* parg = barg + 2 * nblocks;
+        hipLaunchKernelGGL(norms_part, dim3(NF_BLOCKS), dim3(256), 0, st, nblocks, bmax, barg, pmax, parg);
+        hipLaunchKernelGGL(norms_final, dim3(1), dim3(256), 0, st, (int64_t)NF_BLOCKS, pmax, parg, out4);
+    } else {
+        hipLaunchKernelGGL(norms_final, dim3(1), dim3(256), 0, st, nblocks, bmax, barg, out4);
+    }
     return hipGetLastError();
 }
 

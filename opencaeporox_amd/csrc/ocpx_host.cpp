@@ -676,7 +676,7 @@ int ctx_create_impl(int nmodel, const ocpx_fluid* fl, const ocpx_sat* sat, const
     ALLOC(c->rowptr, c->nb + 1); ALLOC(c->colind, c->nnzb); ALLOC(c->tslot, c->nnzb); ALLOC(c->nbr_conn, c->nnzb);
     ALLOC(c->val, (size_t)c->nnzb * B * B); ALLOC(c->rhs, (size_t)c->nb * B); ALLOC(c->resAbs, (size_t)c->nb * B);
     const int64_t nblk = res_asm_blocks(c->nc, c->nb);
-    ALLOC(c->bmax, 2 * nblk); ALLOC(c->barg, 2 * nblk); ALLOC(c->norms4, 4);
+    ALLOC(c->bmax, 2 * nblk + norms_scratch_len()); ALLOC(c->barg, 2 * nblk + norms_scratch_len()); ALLOC(c->norms4, 4);
     ALLOC(c->lam, (size_t)c->nb * B); ALLOC(c->out, (size_t)c->nb * B);
     ALLOC(c->gT, c->nconn); ALLOC(c->gV, c->nb);
     const std::vector<int32_t> ord =

@@ -156,7 +156,8 @@ hipError_t run_tail(int NC, const DevFluid* f, const TailIO& io, hipStream_t st)
 
 // Connection record of a cell, aux_len(b, nc) doubles at aux + n * aux_len
 // (written by krpc_aux, read by the Jacobian assembly):
-//   [8j, 8j + 8)            phase j: rho, Pj, xi, kr, mu, exists (1/0), lambda, depth
+//   [8j, 8j + 8)            phase j: rho, Pj, xi, kr, mu, exists (0 no, 1 yes, 2 yes and some dx_ij/dX is not 0),
+//                           lambda, depth
 //   [24 + 3bj, 24 + 3b(j+1)) phase j: dlambda[b], dPj[b], drho[b] over the primary variables
 //   [24 + 9b + nc j, ...)    phase j: x_ij, i < nc
 // Even length keeps every record 16-byte aligned.
@@ -200,8 +201,9 @@ hipError_t run_krpc_rock(const DevSat* s, const DevRock* r, const CellIO& c, hip
 hipError_t run_res_asm(int nc, const CellIO& c, const ConnIO& cn, const BsrIO& bsr, double dt,
                        bool do_res, bool do_jac, double* res, double* blockmax, int64_t* blockarg,
                        hipStream_t st);
-hipError_t run_norms_final(int64_t nblocks, const double* blockmax, const int64_t* blockarg,
-                           double* out4, hipStream_t st);
+// blockmax and blockarg hold 2 nblocks + norms_scratch_len() entries
+hipError_t run_norms_final(int64_t nblocks, double* blockmax, int64_t* blockarg, double* out4, hipStream_t st);
+int norms_scratch_len();
 // norms of the residual in res (-R) into blockmax/blockarg (res_asm_blocks(nc, nb) blocks)
 hipError_t run_res_norms(int nc, const CellIO& c, const double* res, double* blockmax, int64_t* blockarg,
                          hipStream_t st);

@@ -65,3 +65,48 @@ def test_empty_grid_is_rejected():
     wl = _cells(0)
     with pytest.raises(OcpxError, match="no cells"):
         IsoTFIM.from_workload(wl)
+
+
+# 1,024 workgroups of the residual kernel, one more, and more than the first
+# reduction's threads; the largest term in the first, a middle or the last cell
+@pytest.mark.parametrize("Nc,nb", [(2, 16384), (6, 8193), (12, 4097), (12, 131077)])
+def test_residual_norms_over_many_workgroups(Nc, nb):
+    wl = _cells(nb, Nc)
+    dev = IsoTFIM.from_workload(wl)
+    dev.CalFlash(BATCHED)
+    dev.CalKrPc()
+    dev.CalRock()
+    for n in (0, nb // 2, nb - 1):
+        lni = wl.state["LNI"].copy().reshape(nb, dev.nc)
+        lni[n] *= 1e4
+        dev.set("LNI", lni)
+        res, (v, iv, w, iw) = dev.CalRes(1.0)
+        r = np.abs(res.reshape(nb, dev.bs))
+        rv = (r / dev.get("ROCKVP")[:, None]).max(axis=1)
+        rn = (r[:, 1:] / dev.get("NT")[:, None]).max(axis=1)
+        assert (iv, iw) == (np.argmax(rv), np.argmax(rn)) and iv == n
+        assert np.isclose(v, rv.max(), rtol=1e-14, atol=0) and np.isclose(w, rn.max(), rtol=1e-14, atol=0)
+    dev.close()
+
+
+@pytest.mark.parametrize("Nc", [2, 6, 12])
+def test_assembly_with_some_composition_derivatives_zero(oracle, Nc):
+    """Phases whose dx_ij/dX are all zero, or all but one entry, beside whole ones."""
+    wl = _clean_grid(seed=50 + Nc, Nc=Nc, nx=5, ny=3, nz=3)
+    dev = IsoTFIM.from_workload(wl)
+    st = state_from_workload(wl)
+    oracle.cal_flash(wl.fluid, st)
+    nc, b = dev.nc, dev.bs
+    rng = np.random.Generator(np.random.PCG64(Nc))
+    X = st.a["DSEC_DPRI"].reshape(dev.nb, -1, b)
+    dx = X[:, 3:3 + 3 * nc].reshape(dev.nb, 3, nc, b)
+    kind = rng.integers(0, 3, (dev.nb, 3))
+    one = np.zeros_like(dx)
+    one[..., nc - 1, b - 1] = 1e-3
+    one[..., 0, 0] = np.where(kind == 1, 0.0, 1e-3)
+    dx[:] = np.where((kind == 0)[..., None, None], 0.0, np.where((kind == 1)[..., None, None], one, dx))
+    X[:, 3:3 + 3 * nc] = dx.reshape(dev.nb, 3 * nc, b)
+    st.a["DSEC_DPRI"] = X.reshape(st.a["DSEC_DPRI"].shape)
+    _upload_flash(dev, st)
+    _compare_assembly(dev, oracle, wl, st, 1.0, f"Nc={Nc}")
+    dev.close()
