@@ -80,12 +80,12 @@ struct StaIO {
                                 //      3 resumed at SplitNR after the split stage, 4 resumed at
                                 //      the restart loop after the split-Newton stage, 5 written out,
                                 //      6 long (taken by the general kernel beside the stages)
-    int32_t* decided;           // [nb] first trial stage 1 found unstable, 4 none
-    int32_t* defer;             // [nb] bit k: trial k queued for its Newton step
-    double* Ytd;                // [nb] Yt of the decided trial
+    bool apart;                 // stage 1 takes a cell's trials on lanes of their own
+    int32_t* stop;              // [nb] first trial found unstable so far, 4 none
+    double* Ytd;                // [4][nb] Yt of a trial stage 1 found unstable
     int32_t* evals;             // [nb] stage-1 fugacity evaluations
     int32_t* its;               // [4][nb] SSM iterations per trial
-    int32_t* item;              // [4][nb] Newton item of a queued trial
+    int32_t* item;              // [4][nb] Newton item of a queued trial, -1 stable, -2 unstable
     double* di;                 // [Nc][nb] phi * z of the feed
     int64_t nr_cap;             // Newton items (4 nb)
     int32_t *nr_cell, *nr_k, *nr_flag, *nr_its, *nr_evals;   // [nr_cap]
@@ -101,8 +101,8 @@ struct StaIO {
 // (stability SSM loops), grid[1] (stability Newton steps), grid[2] (split
 // SSM loops) and grid[3] (split Newton steps) 64-lane blocks
 hipError_t run_pe_sta(int NC, const DevFluid* f, const PeIO& io, const StaIO& s, const int* grid, hipStream_t st);
-// before run_pe_sta: zero the stage counters and, with s.long_evals, mark the
-// long cells and list them
+// before run_pe_sta: zero the stage counters, mark no trial unstable and, with
+// s.long_evals, mark the long cells and list them
 hipError_t run_pe_sta_prep(const StaIO& s, int64_t nb, hipStream_t st);
 // resident blocks per compute unit of the stability SSM (which = 0), Newton
 // (1), split (2) and split-Newton (3) stages

@@ -7,7 +7,8 @@
 // with Yt > 1 + eYt declares the feed unstable.  The SSM loops are most of a
 // flash's work, and they share one short body.  So:
 //
-//   stage 1  pe_sta_ssm   persistent lanes, one cell each: SkipPSA's flash
+//   stage 1  pe_sta_ssm   persistent lanes, one cell each (few cells: one trial
+//                         of a cell each, apart): SkipPSA's flash
 //                         type, the feed's ln phi, then the trials' SSM loops
 //                         only.  A trial whose residual is already below
 //                         NRSTA's tolerance needs no Newton step and is
@@ -26,11 +27,13 @@
 //   stage 4  pe_sta_split persistent lanes, one unstable cell each:
 //                         SplitSSM2's first pass (Wilson K, RachfordRice2,
 //                         UpdateXRR, ln phi of both phases, K update) to
-//                         SSMSP's tolerance or cap.  The general kernel
+//                         SSMSP's tolerance or cap (pe_sta_split2: two lanes
+//                         per cell, one per phase).  The general kernel
 //                         resumes every such cell at SplitNR and carries on
 //                         (Newton steps, CheckSplit, the restart loop).
 //   stage 5  pe_sta_snr   (with it) persistent lanes over the cells stage 4
-//                         leaves: SplitNR and CheckSplit, results written
+//                         leaves (pe_sta_snr2: two lanes per cell, one per
+//                         phase): SplitNR and CheckSplit, results written
 //                         out; a cell whose Newton steps do not converge
 //                         goes to the general kernel, which resumes it at
 //                         the restart loop.
@@ -45,7 +48,8 @@
 namespace ocpx {
 namespace sta {
 
-constexpr int NONE = 4;          // decided: no trial found unstable
+constexpr int NONE = 4;                            // no trial found unstable
+constexpr int IT_STABLE = -1, IT_UNSTABLE = -2;    // s.item of a trial that needs no Newton step
 #ifndef STA_WAVES
 #define STA_WAVES 2               // stage-1 wavefronts per SIMD the register budget targets
 #endif
@@ -145,8 +149,8 @@ enum : int { S_IDLE = 0, S_FEED, S_START, S_SSM };
 // ln phi at y (src/OCPEoS.cpp:68-124, 199-214 in log form) with the cell's
 // sqrt(Ai) in registers and Bi = bT P / T formed where used, so a lane holds
 // only what the SSM loop carries
-template <int NC, class F>
-DEV void lean_lnphi(const F& f, const double* sA, double PT, const double* y, double* ev)
+template <int NC, class F, class Cubic>
+DEV void lean_lnphi(const F& f, const double* sA, double PT, const double* y, double* ev, Cubic cubic)
 {
     double w[NC];
     UNROLL for (int k = 0; k < NC; k++) w[k] = sA[k] * y[k];
@@ -158,7 +162,7 @@ DEV void lean_lnphi(const F& f, const double* sA, double PT, const double* y, do
         A += y[i] * ev[i];
         B += (f.bT[i] * PT) * y[i];
     }
-    const double Z = pr_z(A, B);
+    const double Z = cubic(A, B);
     const double lz = log(Z - B);
     const double lg = log((Z + D1 * B) / (Z + D2 * B));
     const double cA = A / (D1 - D2) / B * lg;
@@ -169,6 +173,12 @@ DEV void lean_lnphi(const F& f, const double* sA, double PT, const double* y, do
     }
 }
 
+template <int NC, class F>
+DEV void lean_lnphi(const F& f, const double* sA, double PT, const double* y, double* ev)
+{
+    lean_lnphi<NC>(f, sA, PT, y, ev, [](double A, double B) { return pr_z(A, B); });
+}
+
 // stage 1: one lane per cell, persistent over the work queue
 template <int NC, bool MULTI>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(STA_WAVES)))
@@ -176,9 +186,10 @@ pe_sta_ssm(const DevFluid* __restrict__ fp, PeIO io, StaIO s)
 {
     const size_t n = io.nb;
     const int lane = __lane_id();
-    int cell = -1, st = S_IDLE, k = 0, iter = 0, decided = NONE, defer = 0;
-    int its[4] = {0, 0, 0, 0};
-    double P = 0, PT = 0, logP = 0, Tk = 0, Yt = 0, Ytd = 0;
+    const bool apart = s.apart;
+    const unsigned total = (unsigned)n << (apart ? 2 : 0);
+    int cell = -1, st = S_IDLE, k = 0, iter = 0, its = 0;
+    double P = 0, PT = 0, logP = 0, Tk = 0, Yt = 0;
     double y[NC], di[NC], lp[NC], sA[NC];
     bool drained = false;
     while (true) {
@@ -193,11 +204,13 @@ pe_sta_ssm(const DevFluid* __restrict__ fp, PeIO io, StaIO s)
             base = __shfl(base, leader);
             bool general = false;
             if (need) {
-                const unsigned idx = base + (unsigned)__popcll(m & ((1ull << lane) - 1ull));
-                if (idx < (unsigned)n && s.long_evals > 0 && s.route[io.qorder ? io.qorder[idx] : (int)idx] == 6) {
+                const unsigned item = base + (unsigned)__popcll(m & ((1ull << lane) - 1ull));
+                const unsigned idx = apart ? item >> 2 : item;
+                if (item < total && s.long_evals > 0 && s.route[io.qorder ? io.qorder[idx] : (int)idx] == 6) {
                     // a long cell: the general kernel beside the stages has it
-                } else if (idx < (unsigned)n) {
+                } else if (item < total) {
                     cell = io.qorder ? io.qorder[idx] : (int)idx;
+                    k = apart ? (int)(item & 3u) : 0;
                     const DevFluid& f0 = fl_of<MULTI>(fp, io, cell);
                     P = io.P[cell];
                     Tk = io.T[cell] + CONV4;                          // SetVarSet :674
@@ -215,9 +228,9 @@ pe_sta_ssm(const DevFluid* __restrict__ fp, PeIO io, StaIO s)
                             sA[i] = sqrt(f0.OA[i] * Pr / (Tr * Tr) * (q * q));
                             y[i] = Ni[i] / Nt;                             // InitNtZ :812-818
                         }
-                        k = 0; iter = 0; decided = NONE; defer = 0;
-                        UNROLL for (int t = 0; t < 4; t++) its[t] = 0;
-                    } else {
+                        iter = 0;
+                        its = 0;
+                    } else if (k == 0) {
                         general = true;
                         s.route[cell] = 0;
                     }
@@ -256,7 +269,7 @@ pe_sta_ssm(const DevFluid* __restrict__ fp, PeIO io, StaIO s)
         if (st == S_FEED) {        // di = phi[Id] x (:403-408), fug[Id] = di P
             UNROLL for (int i = 0; i < NC; i++) {
                 di[i] = exp(ev[i]) * y[i];
-                s.di[(size_t)i * n + cell] = di[i];
+                if (k == 0) s.di[(size_t)i * n + cell] = di[i];
             }
             st = S_START;
         } else {
@@ -281,33 +294,37 @@ pe_sta_ssm(const DevFluid* __restrict__ fp, PeIO io, StaIO s)
                 if (Se > f.SSMsta_tol2) st = S_SSM;
                 else trial_end = true;
             } else {
-                its[k]++;
-                if (!(Se > f.SSMsta_tol2 && ++iter <= f.SSMsta_maxIt)) trial_end = true;
+                its++;
+                // behind a trial found unstable meanwhile: not used, given up
+                if (apart && k > 0 && (its & 7) == 0 &&
+                    __hip_atomic_load(&s.stop[cell], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < k)
+                    st = S_IDLE;
+                else if (!(Se > f.SSMsta_tol2 && ++iter <= f.SSMsta_maxIt)) trial_end = true;
             }
         }
         if (trial_end) {
             // StableNR (:478-488): its residual is the last SSM residual
-            bool done = false;
+            bool done = apart;
+            int item = IT_STABLE;
             if (sqrt(Se) > f.NRsta_tol) {
-                defer |= 1 << k;
                 const unsigned q = atomicAdd(s.ncount, 1u);
                 s.nr_cell[q] = cell;
                 s.nr_k[q] = k;
                 s.nr_Yt[q] = Yt;
                 UNROLL for (int i = 0; i < NC; i++) s.nr_y[(size_t)i * s.nr_cap + q] = y[i];
-                s.item[(size_t)k * n + cell] = (int32_t)q;
+                item = (int)q;
             } else if (Yt > 1 + f.eYt) {                  // flag && Yt > 1 + eYt (:463)
-                decided = k;
-                Ytd = Yt;
+                item = IT_UNSTABLE;
+                if (apart) atomicMin(&s.stop[cell], k);
+                s.Ytd[(size_t)k * n + cell] = Yt;
                 done = true;
             }
+            s.item[(size_t)k * n + cell] = item;
+            s.its[(size_t)k * n + cell] = its;
+            its = 0;
             if (!done && ++k == 4) done = true;
             if (done) {
                 s.route[cell] = 1;
-                s.decided[cell] = decided;
-                s.defer[cell] = defer;
-                s.Ytd[cell] = Ytd;
-                UNROLL for (int t = 0; t < 4; t++) s.its[(size_t)t * n + cell] = its[t];
                 st = S_IDLE;
             } else {
                 st = S_START;
@@ -350,7 +367,12 @@ __global__ void __launch_bounds__(64) pe_sta_nr(const DevFluid* __restrict__ fp,
             base = __shfl(base, leader);
             if (need) {
                 const unsigned idx = base + (unsigned)__popcll(m & ((1ull << lane) - 1ull));
-                if (idx < total) {
+                bool behind = false;                 // a trial behind one stage 1 found unstable is not used
+                if (idx < total && s.apart) {
+                    const int c = s.nr_cell[idx], k = s.nr_k[idx];
+                    for (int t = 0; t < k; t++) behind = behind || s.item[(size_t)t * n + c] == IT_UNSTABLE;
+                }
+                if (idx < total && !behind) {
                     q = idx;
                     cell = s.nr_cell[q];
                     const DevFluid& f = fl_of<MULTI>(fp, io, cell);
@@ -374,12 +396,15 @@ __global__ void __launch_bounds__(64) pe_sta_nr(const DevFluid* __restrict__ fp,
                     iter = 0;
                     flag = 1;
                     busy = true;
-                } else {
+                } else if (!behind) {
                     drained = true;
                 }
             }
         }
-        if (!__any(busy)) break;
+        if (!__any(busy)) {
+            if (!__any(!drained)) break;
+            continue;
+        }
         if (busy) {
             const DevFluid& f = fl_of<MULTI>(fp, io, cell);
             bool fin = false;
@@ -441,18 +466,16 @@ __global__ void __launch_bounds__(256) pe_sta_join(const DevFluid* __restrict__ 
     bool split = false;
     if (cell < (int64_t)n && s.route[cell] == 1) {
         const DevFluid& f = MULTI ? fp[io.mid[cell]] : *fp;
-        const int dec = s.decided[cell], def = s.defer[cell];
         int kstar = NONE;
         double Yt = 0;
         int c0 = 0, c1 = 0, c5 = 1, c6 = 0;      // c5: the feed's evaluation
         for (int k = 0; k < 4; k++) {
-            if (k > dec) break;
-            const int it = s.its[(size_t)k * n + cell];
+            const int it = s.its[(size_t)k * n + cell], item = s.item[(size_t)k * n + cell];
             c0 += it;
             c5 += 1 + it;
-            if (k == dec) { kstar = k; Yt = s.Ytd[cell]; break; }
-            if (def & (1 << k)) {
-                const unsigned q = (unsigned)s.item[(size_t)k * n + cell];
+            if (item == IT_UNSTABLE) { kstar = k; Yt = s.Ytd[(size_t)k * n + cell]; break; }
+            if (item != IT_STABLE) {
+                const unsigned q = (unsigned)item;
                 const int nit = s.nr_its[q];
                 c1 += nit;
                 c5 += s.nr_evals[q];
@@ -620,6 +643,181 @@ pe_sta_split(const DevFluid* __restrict__ fp, PeIO io, StaIO s)
     }
 }
 
+// pr_z (ocpx_dev.hpp) in a context of several models, bit for bit as the split's
+// two evaluations on one lane contracted the cubic's constant term: phase 0
+// rounds the second product of the sum, phase 1 the first
+DEV double pr_z_phase(double A, double B, bool ph1)
+{
+    const double a = (D1 + D2 - 1) * B - 1;
+    const double b = A + D1 * D2 * B * B - (D1 + D2) * B * (B + 1);
+    const double k = D1 * D2 * B * B;
+    const double c = -(ph1 ? fma(k, B + 1, A * B) : fma(A, B, k * (B + 1)));
+    const double Q = (a * a - 3 * b) / 9;
+    const double R = (2 * a * a * a - 9 * a * b + 27 * c) / 54;
+    const double Q3 = Q * Q * Q;
+    const double M = R * R - Q3;
+    if (M <= 0) {
+        const double th = acos(R / sqrt(Q3));
+        const double sq = -2 * sqrt(Q);
+        double z0 = polish(sq * cos(th / 3) - a / 3, a, b, c);
+        double z1 = polish(sq * cos((th + 2 * PI_REF) / 3) - a / 3, a, b, c);
+        double z2 = polish(sq * cos((th - 2 * PI_REF) / 3) - a / 3, a, b, c);
+        const double lo = fmin(z0, fmin(z1, z2));
+        const double hi = fmax(z0, fmax(z1, z2));
+        const double dG = (hi - lo) + log((lo - B) / (hi - B)) -
+                          A / (B * (D2 - D1)) *
+                          log((lo + D1 * B) * (hi + D2 * B) / ((lo + D2 * B) * (hi + D1 * B)));
+        return dG > 0 ? lo : hi;
+    }
+    const double sM = sqrt(M);
+    const double t1 = -R + sM, t2 = R + sM;
+    const double S = copysign(cbrt(fabs(t1)), t1) * (t1 != 0);
+    const double T = -copysign(cbrt(fabs(t2)), t2) * (t2 != 0);
+    return polish(S + T - a / 3, a, b, c);
+}
+
+// the other lane of the pair's value
+__device__ __forceinline__ double pair_other(double v)
+{
+    const long long u = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(u & 0xffffffffll), 0xB1, 0xF, 0xF, false);    // quad_perm [1,0,3,2]
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), 0xB1, 0xF, 0xF, false);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+
+// stage 4 with two lanes per cell: both follow the cell, the even one works out
+// ln phi of x0, the odd one that of x1.  Bound by the instructions of the
+// longest cell's iterations.  Nc = 6, 500,000 cells: 3.2 -> 2.5 ms; Nc = 12,
+// about 9,000 cells: 5.3 -> 3.1 ms.
+template <int NC, bool MULTI>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(SPLIT_WAVES)))
+pe_sta_split2(const DevFluid* __restrict__ fp, PeIO io, StaIO s)
+{
+    const size_t n = io.nb;
+    const int lane = __lane_id();
+    const unsigned total = *s.scount;
+    const bool ph1 = lane & 1;
+    int cell = -1, iter = 0, maxIt = 0, rr = 0;
+    bool busy = false, drained = false;
+    double P = 0, PT = 0, tol2 = 0, nu = 0;
+    double z[NC], K[NC], sA[NC];
+    while (true) {
+        while (true) {
+            const bool need = !busy && !drained;
+            const unsigned long long m = __ballot(need) & 0x5555555555555555ull;     // one lane of each pair
+            if (!m) break;
+            const int leader = __ffsll((long long)m) - 1;
+            unsigned base = 0;
+            if (lane == leader) base = atomicAdd(s.shead, (unsigned)__popcll(m));
+            base = __shfl(base, leader);
+            if (need) {
+                const unsigned idx = base + (unsigned)__popcll(m & ((1ull << (lane & ~1)) - 1ull));
+                if (idx < total) {
+                    cell = s.slist[idx];
+                    const DevFluid& f0 = fl_of<MULTI>(fp, io, cell);
+                    P = io.P[cell];
+                    const double Tk = io.T[cell] + CONV4, logP = log(P);
+                    PT = P / Tk;
+                    double Nt = 0;
+                    UNROLL for (int i = 0; i < NC; i++) { z[i] = io.Ni[(size_t)i * n + cell]; Nt += z[i]; }
+                    UNROLL for (int i = 0; i < NC; i++) {
+                        z[i] = z[i] / Nt;
+                        const double Pr = P / f0.Pc[i], Tr = Tk / f0.Tc[i];
+                        const double q = 1 + f0.mw[i] * (1 - sqrt(Tr));
+                        sA[i] = sqrt(f0.OA[i] * Pr / (Tr * Tr) * (q * q));
+                        K[i] = exp(f0.logPc[i] - logP + f0.kwA[i] * (1 - f0.Tc[i] / Tk));
+                    }
+                    tol2 = f0.SSMsp_tol2;
+                    maxIt = f0.SSMsp_maxIt;
+                    if (s.rs_Yt[cell] < 1.1) {
+                        tol2 *= 1E-1;
+                        maxIt *= 2;
+                    }
+                    iter = 0;
+                    rr = 0;
+                    busy = true;
+                } else {
+                    drained = true;
+                }
+            }
+        }
+        if (!__any(busy)) break;
+        if (!busy) continue;
+
+        const DevFluid& f = fl_of<MULTI>(fp, io, cell);
+        {   // RachfordRice2 on K
+            double Kmin = K[0], Kmax = K[0];
+            UNROLL for (int i = 1; i < NC; i++) { Kmin = fmin(Kmin, K[i]); Kmax = fmax(Kmax, K[i]); }
+            const double numin = 1 / (1 - Kmax), numax = 1 / (1 - Kmin);
+            nu = 0.5 * (numin + numax);
+            int it = 0;
+            while (true) {
+                double rj = 0, J = 0;
+                UNROLL for (int i = 0; i < NC; i++) {
+                    const double km = K[i] - 1;
+                    const double t = 1 / (1 + nu * km);
+                    rj += z[i] * km * t;
+                    J -= z[i] * km * km * t * t;
+                }
+                if (fabs(rj) < f.RR_tol || it > f.RR_maxIt) break;
+                const double d = -rj / J, tn = nu + d;
+                if (tn < numax && tn > numin) nu = tn;
+                else nu = d > 0 ? (nu + numax) / 2 : (nu + numin) / 2;
+                it++;
+            }
+            rr += it;
+        }
+        double x[NC], l[NC], l0[NC], l1[NC];
+        UNROLL for (int i = 0; i < NC; i++) {
+            const double x1 = z[i] / (1 + nu * (K[i] - 1)), x0 = K[i] * x1;
+            x[i] = ph1 ? x1 : x0;
+        }
+        if constexpr (MULTI)
+            lean_lnphi<NC>(fp[io.mid[cell]], sA, PT, x, l, [ph1](double A, double B) { return pr_z_phase(A, B, ph1); });
+        else lean_lnphi<NC>(*cfl(fp), sA, PT, x, l);
+        double phi[2][NC];
+        UNROLL for (int i = 0; i < NC; i++) {
+            const double e = exp(l[i]), lo = pair_other(l[i]), eo = pair_other(e);
+            l0[i] = ph1 ? lo : l[i];
+            l1[i] = ph1 ? l[i] : lo;
+            phi[0][i] = ph1 ? eo : e;
+            phi[1][i] = ph1 ? e : eo;
+        }
+        iter++;
+        double Se = 0;
+        UNROLL for (int i = 0; i < NC; i++) {
+            const double x1 = z[i] / (1 + nu * (K[i] - 1)), x0 = K[i] * x1;
+            const double q = (phi[1][i] * x1 * P) / (phi[0][i] * x0 * P) - 1;
+            Se += q * q;
+        }
+        bool last, conv = true;
+        if (iter > maxIt) { conv = false; last = true; }
+        else last = !(Se > tol2);
+        if (last && !ph1) {     // x0, x1 of this iteration's K, then the updated K
+            UNROLL for (int i = 0; i < NC; i++) {
+                const double x1 = z[i] / (1 + nu * (K[i] - 1)), x0 = K[i] * x1;
+                s.rs_v[(size_t)(0 * NC + i) * n + cell] = x0;
+                s.rs_v[(size_t)(1 * NC + i) * n + cell] = x1;
+                s.rs_v[(size_t)(3 * NC + i) * n + cell] = l0[i];
+                s.rs_v[(size_t)(4 * NC + i) * n + cell] = l1[i];
+            }
+        }
+        UNROLL for (int i = 0; i < NC; i++) K[i] = phi[1][i] / phi[0][i];
+        if (last && !ph1) {
+            UNROLL for (int i = 0; i < NC; i++) s.rs_v[(size_t)(2 * NC + i) * n + cell] = K[i];
+            s.rs_nu[cell] = nu;
+            s.rs_cnt[(size_t)2 * n + cell] += 2 * iter;
+            s.rs_cnt[(size_t)4 * n + cell] = iter;
+            s.rs_cnt[(size_t)5 * n + cell] = rr;
+            s.rs_cnt[(size_t)6 * n + cell] = conv ? 1 : 0;
+            s.route[cell] = 3;
+        }
+        if (last) busy = false;
+        if (s.snr) append(last && !ph1, s.tcount, s.tlist, cell);
+        else append(last && !ph1, s.gcount, s.glist, cell);
+    }
+}
+
 // stage 5: SplitNR (:805-897, AssembleJmatSP :911-937, CalStepNRsp
 // :939-957) from what stage 4 left, then, when it converges, CheckSplit
 // (:960-1010) and the cell's results; otherwise PhaseSplit's restart loop
@@ -781,18 +979,206 @@ pe_sta_snr(const DevFluid* __restrict__ fp, PeIO io, StaIO s)
     }
 }
 
+// lnfn_entry (ocpx_dev.hpp) of the lane's phase, bit for bit as pe_sta_snr's
+// contraction forms the two: phase 0 rounds the Bi / B term before the addition
+// and phase 1 the 1 / C one
+template <int NC>
+DEV double lnfn_of_phase(const DevFluid& f, const EosCell<NC>& e, const EosMix<NC>& m, const LnfN<NC>& d,
+                         const double* x, double P, double nt, int i, int k, bool ph1)
+{
+    const double A = m.A, B = m.B, Z = m.Z;
+    const double ZB = Z - B;
+    const double G = (Z + D1 * B) / (Z + D2 * B);
+    const double si = m.s[i];
+    const double E = -A / ((D1 - D2) * B) * (2 * si / A - e.Bi[i] / B);
+    const double aik = f.omk[i * OCPX_NCMAX + k] * e.sA[i] * e.sA[k];
+    const double C = x[i] * P / ZB;
+    const double Cn = P / ZB / ZB * (ZB / nt * ((i == k ? 1.0 : 0.0) - x[i]) - x[i] * (d.Zn[k] - d.Bn[k]));
+    const double iC = 1 / C, bi = e.Bi[i] / B;
+    const double dz = d.Zn[k] - (e.Bi[k] - B) * (Z - 1) / (nt * B);
+    const double Gn = (D1 - D2) / ((Z + D2 * B) * (Z + D2 * B)) * (d.Bn[k] * Z - d.Zn[k] * B);
+    double En = -1 / (D1 - D2) / (B * B) *
+                (2 * (B * aik / nt + d.Bn[k] * (e.Bi[i] * A / B - si)) - d.An[k] * e.Bi[i] - A * e.Bi[i] / nt);
+    En -= E / nt;
+    const double c0 = fma(iC, Cn, bi * dz), c1 = fma(bi, dz, iC * Cn);
+    return (ph1 ? c1 : c0) + En * log(G) + E / G * Gn;
+}
+
+// stage 5 with two lanes per cell: both follow the cell, each works out its
+// phase's part of the Newton matrix and ln phi, and the matrix is solved on
+// both.  Half the code of pe_sta_snr, which does not fit the instruction cache.
+// Nc = 6, 500,000 cells: 1.67 -> 1.21 ms; Nc = 12, about 9,000 cells: 4.1 -> 2.5 ms.
+template <int NC, bool MULTI>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(SNR_WAVES)))
+pe_sta_snr2(const DevFluid* __restrict__ fp, PeIO io, StaIO s)
+{
+    const size_t n = io.nb;
+    const int lane = __lane_id();
+    const unsigned total = *s.tcount;
+    const bool ph1 = lane & 1;
+    int cell = -1, iter = 0;
+    bool busy = false, drained = false, newton = false, conv = false;
+    double P = 0, nu0 = 0, eNR0 = 0;
+    double z[NC], a1[NC], a2[NC], a3[NC], a5[NC];
+    EosCell<NC> ec;
+    while (true) {
+        while (true) {
+            const bool need = !busy && !drained;
+            const unsigned long long m = __ballot(need) & 0x5555555555555555ull;     // one lane of each pair
+            if (!m) break;
+            const int leader = __ffsll((long long)m) - 1;
+            unsigned base = 0;
+            if (lane == leader) base = atomicAdd(s.thead, (unsigned)__popcll(m));
+            base = __shfl(base, leader);
+            if (need) {
+                const unsigned idx = base + (unsigned)__popcll(m & ((1ull << (lane & ~1)) - 1ull));
+                if (idx < total) {
+                    cell = s.tlist[idx];
+                    const DevFluid& f0 = fl_of<MULTI>(fp, io, cell);
+                    P = io.P[cell];
+                    eos_cell<NC>(f0, P, io.T[cell] + CONV4, ec);
+                    double Nt = 0;
+                    UNROLL for (int i = 0; i < NC; i++) { z[i] = io.Ni[(size_t)i * n + cell]; Nt += z[i]; }
+                    UNROLL for (int i = 0; i < NC; i++) z[i] = z[i] / Nt;
+                    nu0 = s.rs_nu[cell];
+                    // SplitNR :807-823: n0 = nu0 x0, resSP = ln(f1 / f0)
+                    double e2 = 0;
+                    UNROLL for (int i = 0; i < NC; i++) {
+                        a2[i] = s.rs_v[(size_t)i * n + cell];
+                        a3[i] = s.rs_v[(size_t)(NC + i) * n + cell];
+                        const double l0 = s.rs_v[(size_t)(3 * NC + i) * n + cell];
+                        const double l1 = s.rs_v[(size_t)(4 * NC + i) * n + cell];
+                        a1[i] = nu0 * a2[i];
+                        a5[i] = log((exp(l1) * a3[i] * P) / (exp(l0) * a2[i] * P));
+                        e2 += a5[i] * a5[i];
+                    }
+                    const double eNR = sqrt(e2);
+                    eNR0 = eNR;
+                    iter = 0;
+                    newton = eNR > f0.NRsp_tol;
+                    conv = !newton && eNR < f0.NRsp_tol;
+                    busy = true;
+                } else {
+                    drained = true;
+                }
+            }
+        }
+        if (!__any(busy)) break;
+        if (!busy) continue;
+
+        bool end = !newton;
+        if (newton) {
+            const DevFluid& f = fl_of<MULTI>(fp, io, cell);
+            const double nu1 = 1 - nu0;
+            double J[NC][NC], rhs[1][NC];
+            {
+                double x[NC];
+                UNROLL for (int i = 0; i < NC; i++) x[i] = ph1 ? a3[i] : a2[i];
+                const double nt = ph1 ? nu1 : nu0;
+                EosMix<NC> m;
+                LnfN<NC> d;
+                eos_mix<NC>(f, ec, x, m);
+                lnfn_prep<NC>(ec, m, nt, d);
+                UNROLL for (int i = 0; i < NC; i++) {
+                    UNROLL for (int k = 0; k <= i; k++) {
+                        const double e = lnfn_of_phase<NC>(f, ec, m, d, x, P, nt, i, k, ph1);
+                        const double v = e + pair_other(e);
+                        J[i][k] = v;
+                        J[k][i] = v;
+                    }
+                    rhs[0][i] = a5[i];
+                }
+            }
+            gauss_solve<NC, 1>(J, rhs);
+            double alpha = 1;                          // CalStepNRsp
+            UNROLL for (int i = 0; i < NC; i++)
+                if (a1[i] + alpha * rhs[0][i] < 0) alpha *= 0.9 * fabs(a1[i] / rhs[0][i]);
+            double nn = 0, en = 0;
+            UNROLL for (int i = 0; i < NC; i++) {
+                const double d = alpha * rhs[0][i];
+                a1[i] += d;
+                nn += a1[i];
+                en += 2 * d * d;
+            }
+            nu0 = nn;
+            const double r0 = 1 / nu0, r1 = 1 / (1 - nu0);
+            UNROLL for (int i = 0; i < NC; i++) {
+                a2[i] = fabs(a1[i] * r0);
+                a3[i] = fabs((z[i] - a1[i]) * r1);
+            }
+            double l[NC], x[NC];
+            {
+                UNROLL for (int i = 0; i < NC; i++) x[i] = ph1 ? a3[i] : a2[i];
+                EosMix<NC> m;
+                eos_mix<NC>(f, ec, x, m);
+                eos_lnphi<NC>(ec, m, l);
+            }
+            double e2 = 0;
+            UNROLL for (int i = 0; i < NC; i++) {
+                const double t = exp(l[i]) * x[i] * P, o = pair_other(t);
+                a5[i] = log((ph1 ? t : o) / (ph1 ? o : t));
+                e2 += a5[i] * a5[i];
+            }
+            const double eNR = sqrt(e2);
+            iter++;
+            if (eNR > eNR0 || iter > f.NRsp_maxIt) end = true;
+            else if (en < 1E-16 * (2.0 * NC) * (2.0 * NC)) { conv = true; end = true; }
+            else if (!(eNR > f.NRsp_tol)) end = true;
+            if (end && eNR < f.NRsp_tol) conv = true;
+        }
+        bool restart = false;
+        if (end) {
+            const int c0 = s.rs_cnt[cell], c1 = s.rs_cnt[n + cell], c5 = s.rs_cnt[2 * n + cell];
+            const int c6 = s.rs_cnt[3 * n + cell], c2 = s.rs_cnt[4 * n + cell], c4 = s.rs_cnt[5 * n + cell];
+            if (ph1) {
+                restart = false;
+            } else if (conv) {                         // CheckSplit, then the results (PhaseEquilibrium :106-111)
+                int NP = 2;
+                const double nuMax = fmax(nu0, 1 - nu0);
+                double eX = 0;
+                UNROLL for (int i = 0; i < NC; i++) eX += (a2[i] - a3[i]) * (a2[i] - a3[i]);
+                if (!(nuMax < 1 && finite_d(eX)) && (!finite_d(eX) || 1 - nuMax < 1E-3)) NP = 1;
+                io.pe_NP[cell] = NP;
+                io.pe_nu[cell] = NP > 1 ? nu0 : 1.0;
+                UNROLL for (int i = 0; i < NC; i++) {
+                    io.pe_x[(size_t)i * n + cell] = NP > 1 ? a2[i] : z[i];
+                    io.pe_x[(size_t)(NC + i) * n + cell] = NP > 1 ? a3[i] : 0.0;
+                }
+                io.ftype_out[cell] = NP > 1 ? 2 : 0;
+                if (io.iters) {
+                    const int cnt[8] = {c0, c1, c2, iter, c4, c5 + 2 * iter, c6 + 2 * iter, c6 + iter};
+                    UNROLL for (int q = 0; q < 8; q++) io.iters[(size_t)q * n + cell] = cnt[q];
+                }
+                s.route[cell] = 5;
+            } else {                                   // the restart loop, in the general kernel
+                s.rs_cnt[2 * n + cell] = c5 + 2 * iter;
+                s.rs_cnt[3 * n + cell] = c6 + 2 * iter;
+                s.rs_cnt[7 * n + cell] = iter;
+                s.route[cell] = 4;
+                restart = true;
+            }
+            busy = false;
+        }
+        append(restart, s.gcount, s.glist, cell);
+    }
+}
+
 __global__ void __launch_bounds__(64) sta_reset(unsigned* c)
 {
     if (threadIdx.x < 10) c[threadIdx.x] = 0;
 }
 
 // route 6 and the list for the cells whose previous flash took more than
-// long_evals fugacity evaluations, route 0 for the others (stage 1 sets theirs)
+// long_evals fugacity evaluations, route 0 for the others (stage 1 sets theirs);
+// no trial found unstable yet
 __global__ void __launch_bounds__(256) sta_pick_long(int64_t nb, StaIO s)
 {
     const int64_t cell = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const bool isl = cell < nb && s.prev_evals[cell] > s.long_evals;
-    if (cell < nb) s.route[cell] = isl ? 6 : 0;
+    const bool isl = s.long_evals > 0 && cell < nb && s.prev_evals[cell] > s.long_evals;
+    if (cell < nb) {
+        s.route[cell] = isl ? 6 : 0;
+        s.stop[cell] = NONE;
+    }
     append(isl, s.lcount, s.llist, (int32_t)cell);
 }
 
@@ -807,18 +1193,37 @@ int blocks_per_cu(int which)
     return e == hipSuccess && b > 0 ? b : 2;
 }
 
+// Stage 1 puts a cell's trials on lanes of their own while they are at most 1.5
+// per lane of the launch: a cell's four SSM loops then end with the longest
+// instead of one after another.  Flash of 33,511 cells at Nc = 5: 5.2 -> 4.6 ms,
+// 9,000 at Nc = 12: 12.0 -> 10.4, 50,000 at Nc = 11: 16.3 -> 16.0; at 65,000
+// cells of Nc = 5 the trials behind an unstable one cost more than it gains
+// (7.2 -> 7.5).
+constexpr int APART_CELLS = 24;
+// Stages 4 and 5 take two lanes per cell while the cells are at most 5 per lane
+// of stage 4's launch.  One iteration then has half the instructions, and long
+// lists still fill the device: 9,000 cells at Nc = 12, 10.4 -> 8.2 ms; 600,000
+// at Nc = 9, 25.9 -> 23.5; a million at Nc = 9 (stages 4 and 5, 12.1 ms on one
+// lane, 13.5 on two) stay on one.
+constexpr int PAIR_CELLS = 320;
+
 template <int NC, bool MULTI>
-hipError_t launch(const DevFluid* f, const PeIO& io, const StaIO& s, const int* grid, hipStream_t st)
+hipError_t launch(const DevFluid* f, const PeIO& io, StaIO s, const int* grid, hipStream_t st)
 {
     if (io.nb == 0) return hipSuccess;
-    const long need = (io.nb + 63) / 64;
-    long g[4];
-    for (int q = 0; q < 4; q++) g[q] = grid[q] < need ? grid[q] : need;
-    hipLaunchKernelGGL((pe_sta_ssm<NC, MULTI>), dim3((unsigned)g[0]), dim3(64), 0, st, f, io, s);
-    hipLaunchKernelGGL((pe_sta_nr<NC, MULTI>), dim3((unsigned)g[1]), dim3(64), 0, st, f, io, s);
-    hipLaunchKernelGGL((pe_sta_join<NC, MULTI>), dim3((unsigned)((io.nb + 255) / 256)), dim3(256), 0, st, f, io, s);
-    if (s.split) hipLaunchKernelGGL((pe_sta_split<NC, MULTI>), dim3((unsigned)g[2]), dim3(64), 0, st, f, io, s);
-    if (s.split && s.snr) hipLaunchKernelGGL((pe_sta_snr<NC, MULTI>), dim3((unsigned)g[3]), dim3(64), 0, st, f, io, s);
+    s.apart = io.nb <= (int64_t)APART_CELLS * grid[0];
+    const bool pair = io.nb <= (int64_t)PAIR_CELLS * grid[2];
+    const int64_t n = io.nb;
+    const int64_t lanes[4] = {s.apart ? 4 * n : n, n, pair ? 2 * n : n, pair ? 2 * n : n};
+    dim3 g[4];
+    for (int q = 0; q < 4; q++) g[q] = dim3((unsigned)(grid[q] < (lanes[q] + 63) / 64 ? grid[q] : (lanes[q] + 63) / 64));
+    hipLaunchKernelGGL((pe_sta_ssm<NC, MULTI>), g[0], dim3(64), 0, st, f, io, s);
+    hipLaunchKernelGGL((pe_sta_nr<NC, MULTI>), g[1], dim3(64), 0, st, f, io, s);
+    hipLaunchKernelGGL((pe_sta_join<NC, MULTI>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, f, io, s);
+    if (s.split && pair) hipLaunchKernelGGL((pe_sta_split2<NC, MULTI>), g[2], dim3(64), 0, st, f, io, s);
+    else if (s.split) hipLaunchKernelGGL((pe_sta_split<NC, MULTI>), g[2], dim3(64), 0, st, f, io, s);
+    if (s.split && s.snr && pair) hipLaunchKernelGGL((pe_sta_snr2<NC, MULTI>), g[3], dim3(64), 0, st, f, io, s);
+    else if (s.split && s.snr) hipLaunchKernelGGL((pe_sta_snr<NC, MULTI>), g[3], dim3(64), 0, st, f, io, s);
     return hipGetLastError();
 }
 
@@ -827,7 +1232,7 @@ hipError_t launch(const DevFluid* f, const PeIO& io, const StaIO& s, const int* 
 hipError_t run_pe_sta_prep(const StaIO& s, int64_t nb, hipStream_t st)
 {
     hipLaunchKernelGGL(sta::sta_reset, dim3(1), dim3(64), 0, st, s.qhead);
-    if (s.long_evals > 0 && nb > 0)
+    if (nb > 0)
         hipLaunchKernelGGL(sta::sta_pick_long, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, st, nb, s);
     return hipGetLastError();
 }

@@ -110,3 +110,26 @@ def test_assembly_with_some_composition_derivatives_zero(oracle, Nc):
     _upload_flash(dev, st)
     _compare_assembly(dev, oracle, wl, st, 1.0, f"Nc={Nc}")
     dev.close()
+
+
+# few cells (trials apart, two lanes per cell), the last and the first number of
+# cells on either side of the rule for the trials, and one lane per cell
+@pytest.mark.parametrize("Nc,nb", [(8, 5), (8, 49152), (3, 49153), (3, 660001)])
+def test_flash_does_not_depend_on_the_number_of_cells(Nc, nb):
+    """The same cells, repeated to nb of them, give the same bits however the stages share them out."""
+    m = min(nb, 1501)
+    wl, _ = W.flash_cells(m, Nc, seed=44 if Nc == 3 else 10 + Nc, P=np.linspace(5.0, 250.0, m))
+    pick = lambda a, n: np.ascontiguousarray(np.asarray(a).reshape(m, -1)[np.arange(n) % m]).ravel()
+    g = wl.grid
+    out = []
+    for n in (m, nb):
+        grid = W.Grid(n, 1, 1, pick(g.v, n), pick(g.depth, n), pick(g.poro, n), np.zeros(0, np.int32),
+                      np.zeros(0, np.int32), np.zeros(0))
+        big = W.Workload(wl.name, wl.fluid, wl.sat, wl.rock, grid, {k: pick(a, n) for k, a in wl.state.items()})
+        dev = IsoTFIM.from_workload(big)
+        dev.CalFlash(BATCHED)
+        out.append({f: dev.get(f).reshape(n, -1) for f in ("ITERS", "PHASEEXIST", "S", "XIJ", "FTYPE_OUT")})
+        dev.close()
+    assert 0 < np.sum(out[0]["PHASEEXIST"][:, :2].sum(axis=1) == 2) < m or m < 100
+    for f in out[0]:
+        assert np.array_equal(out[1][f], out[0][f][np.arange(nb) % m]), f
