@@ -291,7 +291,8 @@ int sta_alloc(ocpx_ctx* c)
     unsigned* cnt = nullptr;
     int rc;
     if ((rc = dalloc(c, &cnt, 16)) || (rc = dalloc(c, &s.glist, n)) || (rc = dalloc(c, &s.route, n)) ||
-        (rc = dalloc(c, &s.stop, n)) || (rc = dalloc(c, &s.Ytd, 4 * n)) ||
+        (rc = dalloc(c, &s.decided, n)) || (rc = dalloc(c, &s.defer, n)) || (rc = dalloc(c, &s.stop, n)) ||
+        (rc = dalloc(c, &s.Ytd, 4 * n)) ||
         (rc = dalloc(c, &s.evals, n)) || (rc = dalloc(c, &s.its, 4 * n)) || (rc = dalloc(c, &s.item, 4 * n)) ||
         (rc = dalloc(c, &s.di, (size_t)c->NC * n)) || (rc = dalloc(c, &s.nr_cell, cap)) ||
         (rc = dalloc(c, &s.nr_k, cap)) || (rc = dalloc(c, &s.nr_flag, cap)) || (rc = dalloc(c, &s.nr_its, cap)) ||

@@ -81,11 +81,13 @@ struct StaIO {
                                 //      the restart loop after the split-Newton stage, 5 written out,
                                 //      6 long (taken by the general kernel beside the stages)
     bool apart;                 // stage 1 takes a cell's trials on lanes of their own
-    int32_t* stop;              // [nb] first trial found unstable so far, 4 none
-    double* Ytd;                // [4][nb] Yt of a trial stage 1 found unstable
+    int32_t* stop;              // [nb] apart: first trial found unstable so far, 4 none
+    int32_t* decided;           // [nb] not apart: first trial stage 1 found unstable, 4 none
+    int32_t* defer;             // [nb] not apart: bit k: trial k queued for its Newton step
+    double* Ytd;                // [nb], apart [4][nb]: Yt of the trial(s) stage 1 found unstable
     int32_t* evals;             // [nb] stage-1 fugacity evaluations
     int32_t* its;               // [4][nb] SSM iterations per trial
-    int32_t* item;              // [4][nb] Newton item of a queued trial, -1 stable, -2 unstable
+    int32_t* item;              // [4][nb] Newton item of a queued trial; apart: else -1 stable, -2 unstable
     double* di;                 // [Nc][nb] phi * z of the feed
     int64_t nr_cap;             // Newton items (4 nb)
     int32_t *nr_cell, *nr_k, *nr_flag, *nr_its, *nr_evals;   // [nr_cap]

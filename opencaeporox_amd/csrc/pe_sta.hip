@@ -179,17 +179,18 @@ DEV void lean_lnphi(const F& f, const double* sA, double PT, const double* y, do
     lean_lnphi<NC>(f, sA, PT, y, ev, [](double A, double B) { return pr_z(A, B); });
 }
 
-// stage 1: one lane per cell, persistent over the work queue
-template <int NC, bool MULTI>
+// stage 1: one lane per cell (apart: per trial of a cell), persistent over the
+// work queue
+template <int NC, bool MULTI, bool apart>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(STA_WAVES)))
 pe_sta_ssm(const DevFluid* __restrict__ fp, PeIO io, StaIO s)
 {
     const size_t n = io.nb;
     const int lane = __lane_id();
-    const bool apart = s.apart;
     const unsigned total = (unsigned)n << (apart ? 2 : 0);
-    int cell = -1, st = S_IDLE, k = 0, iter = 0, its = 0;
-    double P = 0, PT = 0, logP = 0, Tk = 0, Yt = 0;
+    int cell = -1, st = S_IDLE, k = 0, iter = 0, decided = NONE, defer = 0;
+    int its[4] = {0, 0, 0, 0};
+    double P = 0, PT = 0, logP = 0, Tk = 0, Yt = 0, Ytd = 0;
     double y[NC], di[NC], lp[NC], sA[NC];
     bool drained = false;
     while (true) {
@@ -210,7 +211,7 @@ pe_sta_ssm(const DevFluid* __restrict__ fp, PeIO io, StaIO s)
                     // a long cell: the general kernel beside the stages has it
                 } else if (item < total) {
                     cell = io.qorder ? io.qorder[idx] : (int)idx;
-                    k = apart ? (int)(item & 3u) : 0;
+                    if constexpr (apart) k = (int)(item & 3u);
                     const DevFluid& f0 = fl_of<MULTI>(fp, io, cell);
                     P = io.P[cell];
                     Tk = io.T[cell] + CONV4;                          // SetVarSet :674
@@ -228,9 +229,10 @@ pe_sta_ssm(const DevFluid* __restrict__ fp, PeIO io, StaIO s)
                             sA[i] = sqrt(f0.OA[i] * Pr / (Tr * Tr) * (q * q));
                             y[i] = Ni[i] / Nt;                             // InitNtZ :812-818
                         }
-                        iter = 0;
-                        its = 0;
-                    } else if (k == 0) {
+                        if constexpr (!apart) k = 0;
+                        iter = 0; decided = NONE; defer = 0;
+                        UNROLL for (int t = 0; t < 4; t++) its[t] = 0;
+                    } else if (!apart || k == 0) {
                         general = true;
                         s.route[cell] = 0;
                     }
@@ -269,7 +271,7 @@ pe_sta_ssm(const DevFluid* __restrict__ fp, PeIO io, StaIO s)
         if (st == S_FEED) {        // di = phi[Id] x (:403-408), fug[Id] = di P
             UNROLL for (int i = 0; i < NC; i++) {
                 di[i] = exp(ev[i]) * y[i];
-                if (k == 0) s.di[(size_t)i * n + cell] = di[i];
+                if (!apart || k == 0) s.di[(size_t)i * n + cell] = di[i];
             }
             st = S_START;
         } else {
@@ -294,9 +296,9 @@ pe_sta_ssm(const DevFluid* __restrict__ fp, PeIO io, StaIO s)
                 if (Se > f.SSMsta_tol2) st = S_SSM;
                 else trial_end = true;
             } else {
-                its++;
+                its[apart ? 0 : k]++;
                 // behind a trial found unstable meanwhile: not used, given up
-                if (apart && k > 0 && (its & 7) == 0 &&
+                if (apart && k > 0 && (its[0] & 7) == 0 &&
                     __hip_atomic_load(&s.stop[cell], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < k)
                     st = S_IDLE;
                 else if (!(Se > f.SSMsta_tol2 && ++iter <= f.SSMsta_maxIt)) trial_end = true;
@@ -305,26 +307,35 @@ pe_sta_ssm(const DevFluid* __restrict__ fp, PeIO io, StaIO s)
         if (trial_end) {
             // StableNR (:478-488): its residual is the last SSM residual
             bool done = apart;
-            int item = IT_STABLE;
             if (sqrt(Se) > f.NRsta_tol) {
+                defer |= 1 << k;
                 const unsigned q = atomicAdd(s.ncount, 1u);
                 s.nr_cell[q] = cell;
                 s.nr_k[q] = k;
                 s.nr_Yt[q] = Yt;
                 UNROLL for (int i = 0; i < NC; i++) s.nr_y[(size_t)i * s.nr_cap + q] = y[i];
-                item = (int)q;
+                s.item[(size_t)k * n + cell] = (int32_t)q;
             } else if (Yt > 1 + f.eYt) {                  // flag && Yt > 1 + eYt (:463)
-                item = IT_UNSTABLE;
-                if (apart) atomicMin(&s.stop[cell], k);
-                s.Ytd[(size_t)k * n + cell] = Yt;
+                decided = k;
+                Ytd = Yt;
                 done = true;
             }
-            s.item[(size_t)k * n + cell] = item;
-            s.its[(size_t)k * n + cell] = its;
-            its = 0;
             if (!done && ++k == 4) done = true;
             if (done) {
                 s.route[cell] = 1;
+                if constexpr (apart) {
+                    s.its[(size_t)k * n + cell] = its[0];
+                    if (decided == k) {
+                        s.Ytd[(size_t)k * n + cell] = Ytd;
+                        atomicMin(&s.stop[cell], k);
+                    }
+                    if (!defer) s.item[(size_t)k * n + cell] = decided == k ? IT_UNSTABLE : IT_STABLE;
+                } else {
+                    s.decided[cell] = decided;
+                    s.defer[cell] = defer;
+                    s.Ytd[cell] = Ytd;
+                    UNROLL for (int t = 0; t < 4; t++) s.its[(size_t)t * n + cell] = its[t];
+                }
                 st = S_IDLE;
             } else {
                 st = S_START;
@@ -469,10 +480,14 @@ __global__ void __launch_bounds__(256) pe_sta_join(const DevFluid* __restrict__ 
         int kstar = NONE;
         double Yt = 0;
         int c0 = 0, c1 = 0, c5 = 1, c6 = 0;      // c5: the feed's evaluation
+        const int dec = s.apart ? NONE : s.decided[cell], def = s.apart ? 0 : s.defer[cell];
         for (int k = 0; k < 4; k++) {
-            const int it = s.its[(size_t)k * n + cell], item = s.item[(size_t)k * n + cell];
+            if (k > dec) break;
+            const int it = s.its[(size_t)k * n + cell];
             c0 += it;
             c5 += 1 + it;
+            if (k == dec) { kstar = k; Yt = s.Ytd[cell]; break; }
+            const int item = s.apart || (def & (1 << k)) ? s.item[(size_t)k * n + cell] : IT_STABLE;
             if (item == IT_UNSTABLE) { kstar = k; Yt = s.Ytd[(size_t)k * n + cell]; break; }
             if (item != IT_STABLE) {
                 const unsigned q = (unsigned)item;
@@ -1186,7 +1201,7 @@ template <int NC, bool MULTI>
 int blocks_per_cu(int which)
 {
     int b = 0;
-    const hipError_t e = which == 0   ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, pe_sta_ssm<NC, MULTI>, 64, 0)
+    const hipError_t e = which == 0   ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, pe_sta_ssm<NC, MULTI, false>, 64, 0)
                          : which == 1 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, pe_sta_nr<NC, MULTI>, 64, 0)
                          : which == 2 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, pe_sta_split<NC, MULTI>, 64, 0)
                                       : hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, pe_sta_snr<NC, MULTI>, 64, 0);
@@ -1217,7 +1232,8 @@ hipError_t launch(const DevFluid* f, const PeIO& io, StaIO s, const int* grid, h
     const int64_t lanes[4] = {s.apart ? 4 * n : n, n, pair ? 2 * n : n, pair ? 2 * n : n};
     dim3 g[4];
     for (int q = 0; q < 4; q++) g[q] = dim3((unsigned)(grid[q] < (lanes[q] + 63) / 64 ? grid[q] : (lanes[q] + 63) / 64));
-    hipLaunchKernelGGL((pe_sta_ssm<NC, MULTI>), g[0], dim3(64), 0, st, f, io, s);
+    if (s.apart) hipLaunchKernelGGL((pe_sta_ssm<NC, MULTI, true>), g[0], dim3(64), 0, st, f, io, s);
+    else hipLaunchKernelGGL((pe_sta_ssm<NC, MULTI, false>), g[0], dim3(64), 0, st, f, io, s);
     hipLaunchKernelGGL((pe_sta_nr<NC, MULTI>), g[1], dim3(64), 0, st, f, io, s);
     hipLaunchKernelGGL((pe_sta_join<NC, MULTI>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, f, io, s);
     if (s.split && pair) hipLaunchKernelGGL((pe_sta_split2<NC, MULTI>), g[2], dim3(64), 0, st, f, io, s);
