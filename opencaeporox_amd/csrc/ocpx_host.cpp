@@ -289,19 +289,24 @@ int sta_alloc(ocpx_ctx* c)
     const int64_t n = c->nb, cap = 4 * c->nb;
     StaIO& s = c->sta;
     unsigned* cnt = nullptr;
-    int rc;
-    if ((rc = dalloc(c, &cnt, 16)) || (rc = dalloc(c, &s.glist, n)) || (rc = dalloc(c, &s.route, n)) ||
-        (rc = dalloc(c, &s.decided, n)) || (rc = dalloc(c, &s.defer, n)) || (rc = dalloc(c, &s.stop, n)) ||
-        (rc = dalloc(c, &s.Ytd, 4 * n)) ||
-        (rc = dalloc(c, &s.evals, n)) || (rc = dalloc(c, &s.its, 4 * n)) || (rc = dalloc(c, &s.item, 4 * n)) ||
-        (rc = dalloc(c, &s.di, (size_t)c->NC * n)) || (rc = dalloc(c, &s.nr_cell, cap)) ||
-        (rc = dalloc(c, &s.nr_k, cap)) || (rc = dalloc(c, &s.nr_flag, cap)) || (rc = dalloc(c, &s.nr_its, cap)) ||
-        (rc = dalloc(c, &s.nr_evals, cap)) || (rc = dalloc(c, &s.nr_Yt, cap)) ||
-        (rc = dalloc(c, &s.nr_y, (size_t)c->NC * cap)) || (rc = dalloc(c, &s.rs_Yt, n)) ||
-        (rc = dalloc(c, &s.rs_cnt, 8 * n)) || (rc = dalloc(c, &s.slist, n)) || (rc = dalloc(c, &s.tlist, n)) ||
-        (rc = dalloc(c, &s.llist, n)) ||
-        (rc = dalloc(c, &s.rs_v, (size_t)5 * c->NC * n)) || (rc = dalloc(c, &s.rs_nu, n)))
-        return rc;
+    // one allocation, zeroed once: a new context's first flash waits for it
+    std::vector<std::pair<void**, size_t>> parts;
+    auto part = [&](auto** p, size_t count) { parts.emplace_back((void**)p, (count * sizeof(**p) + 255) & ~(size_t)255); };
+    part(&cnt, 16);
+    part(&s.glist, n); part(&s.route, n); part(&s.decided, n); part(&s.defer, n); part(&s.stop, n); part(&s.Ytd, 4 * n);
+    part(&s.evals, n); part(&s.its, 4 * n); part(&s.item, 4 * n); part(&s.di, (size_t)c->NC * n);
+    part(&s.nr_cell, cap); part(&s.nr_k, cap); part(&s.nr_flag, cap); part(&s.nr_its, cap); part(&s.nr_evals, cap);
+    part(&s.nr_Yt, cap); part(&s.nr_y, (size_t)c->NC * cap); part(&s.rs_Yt, n); part(&s.rs_cnt, 8 * n);
+    part(&s.slist, n); part(&s.tlist, n); part(&s.llist, n); part(&s.rs_v, (size_t)5 * c->NC * n); part(&s.rs_nu, n);
+    size_t bytes = 0;
+    for (const auto& q : parts) bytes += q.second;
+    char* slab = nullptr;
+    const int rc = dalloc(c, &slab, bytes);
+    if (rc) return rc;
+    for (const auto& q : parts) {
+        *q.first = slab;
+        slab += q.second;
+    }
     s.qhead = cnt;
     s.gcount = cnt + 1;
     s.ncount = cnt + 2;
