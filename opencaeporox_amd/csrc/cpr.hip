@@ -616,6 +616,8 @@ unsigned grid256(int64_t n) { return (unsigned)((n + 255) / 256); }
 }  // namespace
 
 // ------------------------------------------------------------- PressureAmg
+// Buffers without host data are zeroed on the stream whose kernels use them: a
+// caller's stream need not be ordered with the default one.  setup() waits once.
 template <class T>
 int PressureAmg::dev(T** p, size_t count, const T* host, std::string& err)
 {
@@ -625,7 +627,7 @@ int PressureAmg::dev(T** p, size_t count, const T* host, std::string& err)
     if (e != hipSuccess) { err = std::string("hipMalloc: ") + hipGetErrorString(e); return -1; }
     mem_.push_back(q);
     if (host) e = hipMemcpy(q, host, count * sizeof(T), hipMemcpyHostToDevice);
-    else e = hipMemset(q, 0, count * sizeof(T));
+    else e = hipMemsetAsync(q, 0, count * sizeof(T), st_);
     if (e != hipSuccess) { err = std::string("hipMemcpy: ") + hipGetErrorString(e); return -1; }
     *p = (T*)q;
     return 0;
@@ -637,8 +639,9 @@ PressureAmg::~PressureAmg()
 }
 
 int PressureAmg::setup(int64_t n, const std::vector<int64_t>& rp, const std::vector<int32_t>& col,
-                       const std::vector<double>& w, std::string& err)
+                       const std::vector<double>& w, hipStream_t st, std::string& err)
 {
+    st_ = st;
     amg::Graph g;
     g.n = n;
     g.rp = rp;
@@ -687,6 +690,8 @@ int PressureAmg::setup(int64_t n, const std::vector<int64_t>& rp, const std::vec
             small_ = l;
         }
     }
+    const hipError_t e = hipStreamSynchronize(st);
+    if (e != hipSuccess) { err = std::string("hipMemset: ") + hipGetErrorString(e); return -1; }
     return 0;
 }
 

@@ -41,9 +41,10 @@ public:
 
     // Hierarchy from the level-0 pattern (block rows of the bulk system:
     // rowptr, col with the diagonal first in each row) and the weight of
-    // every off-diagonal slot (its connection's transmissibility).
+    // every off-diagonal slot (its connection's transmissibility).  Buffers are
+    // zeroed on st and ready on return.
     int setup(int64_t n, const std::vector<int64_t>& rp, const std::vector<int32_t>& col,
-              const std::vector<double>& w, std::string& err);
+              const std::vector<double>& w, hipStream_t st, std::string& err);
     bool ready() const { return !lv_.empty(); }
     int levels() const { return (int)lv_.size(); }
     int64_t rows(int l) const { return lv_[l].n; }
@@ -81,6 +82,7 @@ private:
     double *lu_ = nullptr, *inv_ = nullptr;  // dense LU and inverse of the coarsest level (DENSE_MAX^2)
     int32_t* piv_ = nullptr;
     std::vector<void*> mem_;
+    hipStream_t st_ = nullptr;               // setup()'s stream
     template <class T>
     int dev(T** p, size_t count, const T* host, std::string& err);
     hipError_t cycle(int l, double* x, hipStream_t st);

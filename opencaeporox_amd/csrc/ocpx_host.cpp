@@ -1390,7 +1390,7 @@ int cpr_setup(ocpx_ctx* c)
         if (nbc[k] >= 0) w[k] = std::fabs(trans[nbc[k]]);
     auto amg = std::make_unique<PressureAmg>();
     std::string err;
-    if (amg->setup(nb, rp, col, w, err)) return fail(c, OCPX_E_NOMEM, "pressure AMG set-up: " + err);
+    if (amg->setup(nb, rp, col, w, c->st, err)) return fail(c, OCPX_E_NOMEM, "pressure AMG set-up: " + err);
     c->amg = std::move(amg);
     if (!c->gs_rows) {
         std::vector<int32_t> rows;

@@ -4,11 +4,14 @@ method) against a direct sparse solve of the same system, the reference's
 solver settings on the heterogeneous grid with and without its five wells,
 and a Newton iteration that stays on the device (assemble -> solve ->
 GetSolution)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
 import scipy.sparse.linalg as spla
 
+from opencaeporox_amd import abi
 from opencaeporox_amd import workload as W
 from opencaeporox_amd.fim import BATCHED, IsoTFIM
 
@@ -186,3 +189,38 @@ def test_cpr_over_grids_and_colours(Nc, dims, odd):
     # 1e-11 on the decoupled residual, cond(J) below 1e5: as the direct-solve test above
     assert true < 1e-9 and err < 1e-6
     dev.close()
+
+
+def test_solve_after_new_transmissibilities_on_a_callers_stream():
+    """New transmissibilities rebuild the pressure hierarchy of a context whose
+    other buffers are in place; on a stream that is not ordered with the default
+    one the solve is that of a fresh context, bit for bit."""
+    rng = np.random.Generator(np.random.PCG64(29))
+    nx, ny, nz, Nc = 23, 19, 11, 4
+    nb = nx * ny * nz
+    k = np.exp(rng.normal(np.log(100.0), 1.0, nb))
+    grid = W.cartesian_grid(nx, ny, nz, 6.096, k, k, 0.1 * k, rng.uniform(0.1, 0.3, nb))
+    fl, rock = W.make_fluid(Nc, 103), W.make_rock()
+    z = np.tile(rng.dirichlet(np.ones(Nc)), (nb, 1))
+    st = W.initial_state(fl, rock, grid, 200.0 + rng.normal(0, 5.0, nb), z, rng)
+    wl = W.Workload("cpr", fl, W.make_sat(), rock, grid, st)
+    stream = C.c_void_p()
+    assert abi.load().hipStreamCreateWithFlags(C.byref(stream), 1) == 0        # hipStreamNonBlocking
+    dev = IsoTFIM.from_workload(wl, stream=stream)
+    dev.UpdateLastTimeStep()
+    T = grid.trans
+    for trans in (T, T * rng.uniform(0.1, 10.0, T.size), T * rng.uniform(0.01, 1.0, T.size)):
+        dev.set_geometry(trans=trans)
+        dev.ResetToLastTimeStep()
+        dev.newton_pass(0.01, BATCHED)
+        u, it, rr = dev.LinearSolve(rtol=1e-10, maxit=200)
+        fresh = IsoTFIM.from_workload(wl)
+        fresh.set_geometry(trans=trans)
+        fresh.UpdateLastTimeStep()
+        fresh.newton_pass(0.01, BATCHED)
+        v, jt, _ = fresh.LinearSolve(rtol=1e-10, maxit=200)
+        assert it == jt > 0 and rr < 1e-10
+        assert np.array_equal(u, v)
+        fresh.close()
+    dev.close()
+    assert abi.load().hipStreamDestroy(stream) == 0

@@ -7,6 +7,7 @@ res_only, res_asm, xcd_chunk, block_norms) and csrc/wells.hip, evaluated for
 every block and lane of their launch grids."""
 import ctypes as C
 import os
+import re
 import subprocess
 
 import numpy as np
@@ -193,3 +194,14 @@ def test_well_indices_in_bounds(lib):
         assert (npf - 1) * nc + nc - 1 < npf * nc
         assert (nb + nw - 1) * B < (nb + nw) * B
         assert ucell.max() * B + B - 1 < nb * B
+
+
+def test_fills_of_device_memory_name_their_stream():
+    """A context may be bound to a stream that is not ordered with the default
+    one, where a fill could land on what the context's kernels wrote since; a
+    synchronous fill of device memory does not wait either."""
+    for name in sorted(os.listdir(CSRC)):
+        if name.endswith((".hip", ".cpp", ".hpp")):
+            with open(os.path.join(CSRC, name)) as f:
+                for k, line in enumerate(f, 1):
+                    assert not re.search(r"hipMemset(D8|D16|D32|2D|3D)?\s*\(", line), f"{name}:{k}: {line.strip()}"
