@@ -29,6 +29,13 @@ def flags():
     return ["-x", "hip", f"--offload-arch={ARCH}", "-O3", "-fPIC", "-std=c++17",
             # packed FP32 instructions are kept off; this code is FP64 anyway
             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+            # scalar constants are formed where they are used and not at the top of a
+            # block: ahead of the instruction that restores EXEC they make the register
+            # allocator put vector copies and spills before it too, for some of the lanes
+            # only (a team-of-8 flash kernel at Nc = 11 lost coefficients that way;
+            # tests/test_kernel_exec.py reads the built code for it).  The kernels' times
+            # are the same with it, and the same bits.
+            "-mllvm", "-huge-size-for-split=0",
             "-Wno-unused-result", "-I", os.path.join(PKG, "..", "include")]
 
 

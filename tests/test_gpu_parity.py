@@ -111,6 +111,9 @@ PE_CASES = [(Nc, m, lanes, stages) for Nc in (3, 4, 5, 9, 12)
                                      (BATCHED, 16, 3), (BATCHED, 4, 2), (BATCHED, 4, 1), (BATCHED, 1, 0),
                                      (BATCHED, 4, 0), (BATCHED, 1, "long"), (BATCHED, 4, "long"))
             if lanes < 8 or (lanes == 8 and Nc >= 5) or (lanes == 16 and Nc >= 9)]
+# and the team kernels of the other component counts
+PE_CASES += [(Nc, BATCHED, lanes, 3) for Nc in (2, 6, 7, 8, 10, 11) for lanes in (4, 8, 16)
+             if lanes < 8 or (lanes == 8 and Nc >= 5) or (lanes == 16 and Nc >= 9)]
 
 
 @pytest.mark.parametrize("Nc,mode,lanes,stages", PE_CASES)
