@@ -296,6 +296,14 @@ int  ocpx_autotune_flash(ocpx_ctx* ctx, double* ms);
  * models every stage reads each cell's own model's fluid. */
 int  ocpx_set_flash_stages(ocpx_ctx* ctx, int on);
 int  ocpx_get_flash_stages(ocpx_ctx* ctx, int32_t* on);
+/* Variants of the flash stages, which share the same arithmetic out
+ * differently.  trials_apart: the stability SSM stage gives each trial of a
+ * cell a lane of its own instead of one lane per cell; lane_pairs: the split
+ * stages take two lanes per cell, one per phase.  -1 (default): by the number
+ * of cells, where each is the faster one; 0: off; 1: on.  The get call returns
+ * what the next staged flash takes (0 or 1). */
+int  ocpx_set_flash_variants(ocpx_ctx* ctx, int32_t trials_apart, int32_t lane_pairs);
+int  ocpx_get_flash_variants(ocpx_ctx* ctx, int32_t* trials_apart, int32_t* lane_pairs);
 /* Long cells of the staged batched flash.  No counterpart in the reference;
  * the same algorithm either way.  Cells whose previous batched flash took more
  * than `evals` fugacity evaluations (ITERS row 5; default 1000, 0 = off) are

@@ -142,6 +142,8 @@ def load(path=None):
         "ocpx_get_linear_solver": (C.c_int, [vp, C.POINTER(i32)]),
         "ocpx_phase_equilibrium_noalloc": (C.c_int, [C.POINTER(Fluid), i64, vp, vp, vp, vp, vp, vp, vp, vp]),
         "ocpx_get_flash_stages": (C.c_int, [vp, C.POINTER(i32)]),
+        "ocpx_set_flash_variants": (C.c_int, [vp, i32, i32]),
+        "ocpx_get_flash_variants": (C.c_int, [vp, C.POINTER(i32), C.POINTER(i32)]),
         "ocpx_timing_enable": (C.c_int, [vp, C.c_int]),
         "ocpx_timing_get": (C.c_int, [vp, C.c_int, C.POINTER(dbl), C.POINTER(i64)]),
         "ocpx_set_wells": (C.c_int, [vp, i32, vp, vp, vp, vp, vp]),

@@ -96,6 +96,7 @@ struct ocpx_ctx {
                                  // the split's first SSM pass, 3 and its Newton steps (pe_sta.hip), 0 none
     bool sta_ready = false;      // the stage buffers are allocated
     StaIO sta{};
+    int var_apart = -1, var_pair = -1;   // variants of the stages: -1 by the number of cells, 0 off, 1 on
     int long_evals = 1000;       // staged flash: cells over this many evaluations last time run beside the stages
     hipStream_t st2 = nullptr;   // the branch that runs them, forked from and joined to st by events
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
@@ -334,6 +335,14 @@ int sta_alloc(ocpx_ctx* c)
 
 TailIO tail_io(ocpx_ctx* c);
 
+// the variants of the stages the next flash takes: the caller's, else the rule's
+void flash_variants(const ocpx_ctx* c, bool* apart, bool* pair)
+{
+    pe_sta_rule(c->nb, c->sta_grid, apart, pair);
+    if (c->var_apart >= 0) *apart = c->var_apart;
+    if (c->var_pair >= 0) *pair = c->var_pair;
+}
+
 // branch_ok: the long cells may run on the context's second stream and the
 // finished cells' tail on its third (off when the context's own stream is
 // itself a branch of a batch capture); tail_follows: launch_tail comes next
@@ -370,6 +379,7 @@ int launch_pe(ocpx_ctx* c, int mode, bool branch_ok = true, bool tail_follows = 
         if (staged) {
             c->sta.split = c->stages >= 2;
             c->sta.snr = c->stages >= 3;
+            flash_variants(c, &c->sta.apart, &c->sta.pair);
             // the cells that took longest last time run beside the stages from the
             // start (their serial Newton and restart work is the flash's critical path)
             const bool branch = branch_ok && c->long_evals > 0 && mode == OCPX_FLASH_BATCHED;
@@ -987,6 +997,25 @@ int ocpx_get_flash_stages(ocpx_ctx* c, int32_t* on)
 {
     if (!c || !on) return OCPX_E_ARG;
     *on = c->stages;
+    return OCPX_OK;
+}
+
+int ocpx_set_flash_variants(ocpx_ctx* c, int32_t trials_apart, int32_t lane_pairs)
+{
+    if (!c || trials_apart < -1 || trials_apart > 1 || lane_pairs < -1 || lane_pairs > 1) return OCPX_E_ARG;
+    if (trials_apart != c->var_apart || lane_pairs != c->var_pair) destroy_graph(c);
+    c->var_apart = trials_apart;
+    c->var_pair = lane_pairs;
+    return OCPX_OK;
+}
+
+int ocpx_get_flash_variants(ocpx_ctx* c, int32_t* trials_apart, int32_t* lane_pairs)
+{
+    if (!c || !trials_apart || !lane_pairs) return OCPX_E_ARG;
+    bool a, p;
+    flash_variants(c, &a, &p);
+    *trials_apart = a;
+    *lane_pairs = p;
     return OCPX_OK;
 }
 

@@ -81,6 +81,7 @@ struct StaIO {
                                 //      the restart loop after the split-Newton stage, 5 written out,
                                 //      6 long (taken by the general kernel beside the stages)
     bool apart;                 // stage 1 takes a cell's trials on lanes of their own
+    bool pair;                  // the split stages take two lanes per cell
     int32_t* stop;              // [nb] apart: first trial found unstable so far, 4 none
     int32_t* decided;           // [nb] not apart: first trial stage 1 found unstable, 4 none
     int32_t* defer;             // [nb] not apart: bit k: trial k queued for its Newton step
@@ -106,6 +107,8 @@ hipError_t run_pe_sta(int NC, const DevFluid* f, const PeIO& io, const StaIO& s,
 // before run_pe_sta: zero the stage counters, mark no trial unstable and, with
 // s.long_evals, mark the long cells and list them
 hipError_t run_pe_sta_prep(const StaIO& s, int64_t nb, hipStream_t st);
+// the variants (StaIO::apart, pair) that are the faster ones for nb cells
+void pe_sta_rule(int64_t nb, const int* grid, bool* apart, bool* pair);
 // resident blocks per compute unit of the stability SSM (which = 0), Newton
 // (1), split (2) and split-Newton (3) stages
 int pe_sta_blocks_per_cu(int NC, int which, bool multi);

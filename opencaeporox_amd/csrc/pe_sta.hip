@@ -1223,22 +1223,20 @@ constexpr int APART_CELLS = 24;
 constexpr int PAIR_CELLS = 320;
 
 template <int NC, bool MULTI>
-hipError_t launch(const DevFluid* f, const PeIO& io, StaIO s, const int* grid, hipStream_t st)
+hipError_t launch(const DevFluid* f, const PeIO& io, const StaIO& s, const int* grid, hipStream_t st)
 {
     if (io.nb == 0) return hipSuccess;
-    s.apart = io.nb <= (int64_t)APART_CELLS * grid[0];
-    const bool pair = io.nb <= (int64_t)PAIR_CELLS * grid[2];
     const int64_t n = io.nb;
-    const int64_t lanes[4] = {s.apart ? 4 * n : n, n, pair ? 2 * n : n, pair ? 2 * n : n};
+    const int64_t lanes[4] = {s.apart ? 4 * n : n, n, s.pair ? 2 * n : n, s.pair ? 2 * n : n};
     dim3 g[4];
     for (int q = 0; q < 4; q++) g[q] = dim3((unsigned)(grid[q] < (lanes[q] + 63) / 64 ? grid[q] : (lanes[q] + 63) / 64));
     if (s.apart) hipLaunchKernelGGL((pe_sta_ssm<NC, MULTI, true>), g[0], dim3(64), 0, st, f, io, s);
     else hipLaunchKernelGGL((pe_sta_ssm<NC, MULTI, false>), g[0], dim3(64), 0, st, f, io, s);
     hipLaunchKernelGGL((pe_sta_nr<NC, MULTI>), g[1], dim3(64), 0, st, f, io, s);
     hipLaunchKernelGGL((pe_sta_join<NC, MULTI>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, f, io, s);
-    if (s.split && pair) hipLaunchKernelGGL((pe_sta_split2<NC, MULTI>), g[2], dim3(64), 0, st, f, io, s);
+    if (s.split && s.pair) hipLaunchKernelGGL((pe_sta_split2<NC, MULTI>), g[2], dim3(64), 0, st, f, io, s);
     else if (s.split) hipLaunchKernelGGL((pe_sta_split<NC, MULTI>), g[2], dim3(64), 0, st, f, io, s);
-    if (s.split && s.snr && pair) hipLaunchKernelGGL((pe_sta_snr2<NC, MULTI>), g[3], dim3(64), 0, st, f, io, s);
+    if (s.split && s.snr && s.pair) hipLaunchKernelGGL((pe_sta_snr2<NC, MULTI>), g[3], dim3(64), 0, st, f, io, s);
     else if (s.split && s.snr) hipLaunchKernelGGL((pe_sta_snr<NC, MULTI>), g[3], dim3(64), 0, st, f, io, s);
     return hipGetLastError();
 }
@@ -1262,6 +1260,12 @@ hipError_t run_pe_sta(int NC, const DevFluid* f, const PeIO& io, const StaIO& s,
 #undef OCPX_CASE
     default: return hipErrorInvalidValue;
     }
+}
+
+void pe_sta_rule(int64_t nb, const int* grid, bool* apart, bool* pair)
+{
+    *apart = nb <= (int64_t)sta::APART_CELLS * grid[0];
+    *pair = nb <= (int64_t)sta::PAIR_CELLS * grid[2];
 }
 
 int pe_sta_blocks_per_cu(int NC, int which, bool multi)

@@ -185,6 +185,19 @@ class IsoTFIM:
         self._chk(self.lib.ocpx_get_flash_stages(self.h, C.byref(v)), "flash stages")
         return v.value
 
+    def set_flash_variants(self, trials_apart=None, lane_pairs=None):
+        """How the stages share their work out: a lane per trial instead of per
+        cell in the stability test, two lanes per cell instead of one in the split
+        (True / False; None: by the number of cells)."""
+        v = [-1 if q is None else int(bool(q)) for q in (trials_apart, lane_pairs)]
+        self._chk(self.lib.ocpx_set_flash_variants(self.h, *v), "flash variants")
+
+    def flash_variants(self):
+        """(trials_apart, lane_pairs) of the next staged flash."""
+        a, p = C.c_int32(), C.c_int32()
+        self._chk(self.lib.ocpx_get_flash_variants(self.h, C.byref(a), C.byref(p)), "flash variants")
+        return bool(a.value), bool(p.value)
+
     def CalFlash(self, mode=PLAIN):
         self._chk(self.lib.ocpx_flash_der(self.h, mode), "flash")
 

@@ -112,24 +112,67 @@ def test_assembly_with_some_composition_derivatives_zero(oracle, Nc):
     dev.close()
 
 
-# few cells (trials apart, two lanes per cell), the last and the first number of
-# cells on either side of the rule for the trials, and one lane per cell
-@pytest.mark.parametrize("Nc,nb", [(8, 5), (8, 49152), (3, 49153), (3, 660001)])
-def test_flash_does_not_depend_on_the_number_of_cells(Nc, nb):
-    """The same cells, repeated to nb of them, give the same bits however the stages share them out."""
-    m = min(nb, 1501)
-    wl, _ = W.flash_cells(m, Nc, seed=44 if Nc == 3 else 10 + Nc, P=np.linspace(5.0, 250.0, m))
-    pick = lambda a, n: np.ascontiguousarray(np.asarray(a).reshape(m, -1)[np.arange(n) % m]).ravel()
+def _repeated(Nc, m, nb):
+    """The first m of 1,501 flash cells, repeated to nb of them."""
+    wl, _ = W.flash_cells(1501, Nc, seed=44 if Nc == 3 else 10 + Nc, P=np.linspace(5.0, 250.0, 1501))
+    pick = lambda a: np.ascontiguousarray(np.asarray(a).reshape(1501, -1)[np.arange(nb) % m]).ravel()
     g = wl.grid
+    grid = W.Grid(nb, 1, 1, pick(g.v), pick(g.depth), pick(g.poro), np.zeros(0, np.int32), np.zeros(0, np.int32),
+                  np.zeros(0))
+    return W.Workload(wl.name, wl.fluid, wl.sat, wl.rock, grid, {k: pick(a) for k, a in wl.state.items()})
+
+
+# a few cells, and the last and the first number of cells on either side of the rules for the trials' lanes
+# and the pairs of lanes, on 256 compute units of two wavefronts per SIMD
+@pytest.mark.parametrize("Nc,nb,variants", [(8, 5, (True, True)), (8, 49152, (True, True)), (8, 49153, (False, True)),
+                                            (3, 49153, (False, True)), (3, 655360, (False, True)),
+                                            (3, 660001, (False, False)), (8, 655361, (False, False))])
+def test_flash_does_not_depend_on_the_number_of_cells(Nc, nb, variants):
+    """The same cells, repeated to nb of them, give the same bits however the stages share them out."""
+    m = 1501
     out = []
     for n in (m, nb):
-        grid = W.Grid(n, 1, 1, pick(g.v, n), pick(g.depth, n), pick(g.poro, n), np.zeros(0, np.int32),
-                      np.zeros(0, np.int32), np.zeros(0))
-        big = W.Workload(wl.name, wl.fluid, wl.sat, wl.rock, grid, {k: pick(a, n) for k, a in wl.state.items()})
-        dev = IsoTFIM.from_workload(big)
+        dev = IsoTFIM.from_workload(_repeated(Nc, m, n))
+        assert dev.flash_variants() == (variants if n == nb else (True, True))
         dev.CalFlash(BATCHED)
         out.append({f: dev.get(f).reshape(n, -1) for f in ("ITERS", "PHASEEXIST", "S", "XIJ", "FTYPE_OUT")})
         dev.close()
-    assert 0 < np.sum(out[0]["PHASEEXIST"][:, :2].sum(axis=1) == 2) < m or m < 100
+    assert 0 < np.sum(out[0]["PHASEEXIST"][:, :2].sum(axis=1) == 2) < m
     for f in out[0]:
         assert np.array_equal(out[1][f], out[0][f][np.arange(nb) % m]), f
+
+
+@pytest.mark.parametrize("several", [False, True])
+@pytest.mark.parametrize("Nc", range(2, 13))
+def test_flash_stage_variants_give_the_same_bits(Nc, several):
+    """Every way the stages share their work out, over all component counts, in
+    contexts of one model and of several, on the first flash and on the one that
+    follows from its phases (the other flash types and the relaxed test)."""
+    n = 6000
+    out = []
+    for apart, pairs in ((False, False), (False, True), (True, False), (True, True)):
+        if several:
+            dev = IsoTFIM.from_workloads([W.flash_cells(n // 3, Nc, seed=s, P=np.linspace(5.0, 250.0, n // 3))[0]
+                                          for s in (44 if Nc == 3 else 10 + Nc, 103, 127)])
+        else:
+            dev = IsoTFIM.from_workload(W.flash_cells(n, Nc, seed=44 if Nc == 3 else 10 + Nc,
+                                                      P=np.linspace(5.0, 250.0, n))[0])
+        dev.set_flash_variants(trials_apart=apart, lane_pairs=pairs)
+        assert dev.flash_variants() == (apart, pairs)
+        got = {}
+        for k in range(2):
+            dev.CalFlash(BATCHED)
+            got.update({(f, k): dev.get(f) for f in ("ITERS", "PHASEEXIST", "S", "XIJ", "FTYPE_OUT", "DSEC_DPRI")})
+            got.update({(f, k): a for f, a in zip(("NP", "nu", "x"), dev.pe_result())})
+        dev.close()
+        out.append(got)
+    it = out[0]["ITERS", 0].reshape(-1, 8)
+    print(f"Nc={Nc}: {np.sum(it[:, 2] > 0)} cells split, {np.sum(it[:, 3] > 0)} with Newton steps")
+    assert np.sum(it[:, 3] > 0) > 100
+    bad = []
+    for v, got in enumerate(out[1:], 1):
+        for f in got:
+            if not np.array_equal(got[f], out[0][f], equal_nan=True):
+                cells = np.any((got[f] != out[0][f]).reshape(n, -1), axis=1)
+                bad.append(f"variant {v} {f}: {np.sum(cells)} cells, first {np.where(cells)[0][:5]}")
+    assert not bad, "\n".join(bad)

@@ -105,11 +105,13 @@ def test_flash_config1(oracle, oracle_fma, mode, lanes):
 # batched mode with every stage (3), the stability and split-SSM stages (2),
 # the stability stages alone (1) and none (0); "long": every stage, on a
 # second flash in which the cells over 150 fugacity evaluations in the first
-# run on the branch beside the stages
+# run on the branch beside the stages; "one lane": every stage with one lane per
+# cell, as contexts of many cells run them
 PE_CASES = [(Nc, m, lanes, stages) for Nc in (3, 4, 5, 9, 12)
             for m, lanes, stages in ((PLAIN, 1, 0), (BATCHED, 1, 3), (BATCHED, 4, 3), (BATCHED, 8, 3),
                                      (BATCHED, 16, 3), (BATCHED, 4, 2), (BATCHED, 4, 1), (BATCHED, 1, 0),
-                                     (BATCHED, 4, 0), (BATCHED, 1, "long"), (BATCHED, 4, "long"))
+                                     (BATCHED, 4, 0), (BATCHED, 1, "long"), (BATCHED, 4, "long"),
+                                     (BATCHED, 4, "one lane"))
             if lanes < 8 or (lanes == 8 and Nc >= 5) or (lanes == 16 and Nc >= 9)]
 # and the team kernels of the other component counts
 PE_CASES += [(Nc, BATCHED, lanes, 3) for Nc in (2, 6, 7, 8, 10, 11) for lanes in (4, 8, 16)
@@ -134,6 +136,9 @@ def test_phase_equilibrium_cells(oracle, oracle_fma, Nc, mode, lanes, stages):
         print(f"Nc={Nc}: {nlong} cells over 150 evaluations go to the branch")
         assert nlong > 10
         dev.set_flash_long(150)
+    elif stages == "one lane":
+        dev.set_flash_variants(trials_apart=False, lane_pairs=False)
+        assert dev.flash_variants() == (False, False)
     else:
         dev.set_flash_stages(stages)
     dev.PhaseEquilibrium(mode)
