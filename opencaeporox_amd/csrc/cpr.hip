@@ -93,6 +93,17 @@ __global__ void __launch_bounds__(256) amg_dinv(int64_t n, const int64_t* __rest
     dinv[i] = d != 0 ? 1 / d : 0.0;
 }
 
+// a level's pattern in V-cycle order, one thread per position
+__global__ void __launch_bounds__(256) amg_sell_fill(int64_t nq, const int64_t* __restrict__ off,
+                                                     const int32_t* __restrict__ row, const int64_t* __restrict__ rp,
+                                                     const int32_t* __restrict__ gci,
+                                                     const int32_t* __restrict__ agg, int32_t* __restrict__ ci,
+                                                     int32_t* __restrict__ cagg, int32_t* __restrict__ src)
+{
+    const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (q < nq) amg::sell_position(q, off, row, rp, gci, agg, ci, cagg, src);
+}
+
 // a level's values in V-cycle order
 __global__ void __launch_bounds__(256) amg_sell(int64_t ne, const int32_t* __restrict__ src,
                                                 const double* __restrict__ a, double* __restrict__ sa)
@@ -668,12 +679,20 @@ int PressureAmg::setup(int64_t n, const std::vector<int64_t>& rp, const std::vec
         amg::sell_layout(g, M, gc.n, S);
         L.nc = gc.n;
         L.nq = (int64_t)S.row.size();
-        L.ne = (int64_t)S.ci.size();
+        L.ne = S.off.back();
         if (dev(&L.gp, M.gp.size(), M.gp.data(), err) || dev(&L.gs, M.gs.size(), M.gs.data(), err) ||
             dev(&L.off, S.off.size(), S.off.data(), err) || dev(&L.row, S.row.size(), S.row.data(), err) ||
-            dev(&L.sci, S.ci.size(), S.ci.data(), err) || dev(&L.cagg, S.cagg.size(), S.cagg.data(), err) ||
-            dev(&L.src, S.src.size(), S.src.data(), err) || dev(&L.sa, (size_t)L.ne, (const double*)nullptr, err))
+            dev(&L.agg, M.agg.size(), M.agg.data(), err) || dev(&L.sci, (size_t)L.ne, (const int32_t*)nullptr, err) ||
+            dev(&L.cagg, (size_t)L.ne, (const int32_t*)nullptr, err) ||
+            dev(&L.src, (size_t)L.ne, (const int32_t*)nullptr, err) ||
+            dev(&L.sa, (size_t)L.ne, (const double*)nullptr, err))
             return -1;
+        hipLaunchKernelGGL(amg_sell_fill, dim3(grid256(L.nq)), dim3(256), 0, st, L.nq, L.off, L.row, L.rp, L.ci,
+                           L.agg, L.sci, L.cagg, L.src);
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess) {
+            err = std::string("amg_sell_fill: ") + hipGetErrorString(e);
+            return -1;
+        }
         lv_.push_back(L);
         g = std::move(gc);
     }
@@ -691,7 +710,7 @@ int PressureAmg::setup(int64_t n, const std::vector<int64_t>& rp, const std::vec
         }
     }
     const hipError_t e = hipStreamSynchronize(st);
-    if (e != hipSuccess) { err = std::string("hipMemset: ") + hipGetErrorString(e); return -1; }
+    if (e != hipSuccess) { err = std::string("hipStreamSynchronize: ") + hipGetErrorString(e); return -1; }
     return 0;
 }
 

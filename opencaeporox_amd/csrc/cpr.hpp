@@ -74,7 +74,7 @@ private:
         // the level's matrix in V-cycle order (amg::Sell); ne entries
         int64_t nc = 0, nq = 0, ne = 0;
         int64_t* off = nullptr;
-        int32_t *row = nullptr, *sci = nullptr, *cagg = nullptr, *src = nullptr;
+        int32_t *row = nullptr, *agg = nullptr, *sci = nullptr, *cagg = nullptr, *src = nullptr;
         double* sa = nullptr;
     };
     std::vector<Level> lv_;

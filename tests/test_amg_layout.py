@@ -52,14 +52,15 @@ void fetch(int64_t* crp, int32_t* cci, double* cw, int32_t* agg, int64_t* gp, in
 int64_t sell_sizes(int64_t* out)
 {
     amg::sell_layout(G, M, GC.n, S);
-    out[0] = (int64_t)S.row.size(); out[1] = (int64_t)S.off.size(); out[2] = (int64_t)S.ci.size();
+    out[0] = (int64_t)S.row.size(); out[1] = (int64_t)S.off.size(); out[2] = S.off.back();
     return 0;
 }
 void sell_fetch(int64_t* off, int32_t* row, int32_t* ci, int32_t* cagg, int32_t* src)
 {
     for (size_t k = 0; k < S.off.size(); k++) off[k] = S.off[k];
     for (size_t k = 0; k < S.row.size(); k++) row[k] = S.row[k];
-    for (size_t k = 0; k < S.ci.size(); k++) { ci[k] = S.ci[k]; cagg[k] = S.cagg[k]; src[k] = S.src[k]; }
+    for (size_t q = 0; q < S.row.size(); q++)
+        amg::sell_position((int64_t)q, S.off.data(), S.row.data(), G.rp.data(), G.ci.data(), M.agg.data(), ci, cagg, src);
 }
 int64_t colors(int64_t n, const int64_t* rp, const int32_t* ci, int32_t* cptr, int32_t* rows)
 {
