@@ -176,3 +176,31 @@ def test_flash_stage_variants_give_the_same_bits(Nc, several):
                 cells = np.any((got[f] != out[0][f]).reshape(n, -1), axis=1)
                 bad.append(f"variant {v} {f}: {np.sum(cells)} cells, first {np.where(cells)[0][:5]}")
     assert not bad, "\n".join(bad)
+
+
+# one cell, less and more than a wavefront, and one cell more or less than the lanes of a dealt queue can hold
+@pytest.mark.parametrize("nb", [1, 63, 65, 1023, 1025, 2049, 5003])
+def test_one_lane_kernel_takes_every_cell_once(nb):
+    """The one-lane kernel deals a short queue out over its wavefronts; the order
+    changes no bits, on the first flash and in longest-first order on the next."""
+    wl = _repeated(6, 1501, nb)
+    ctx = []
+    for mode, longest in ((PLAIN, False), (BATCHED, False), (BATCHED, True)):
+        dev = IsoTFIM.from_workload(wl)
+        dev.set_flash_mapping(1)
+        dev.set_flash_stages(False)
+        dev.set_flash_queue_order(longest)
+        dev.UpdateLastTimeStep()
+        ctx.append((dev, mode))
+    for k in range(2):
+        out = []
+        for dev, mode in ctx:
+            dev.CalFlash(mode)
+            out.append([dev.get(f) for f in ("FTYPE_OUT", "PHASEEXIST", "S", "XIJ", "DSEC_DPRI")])
+        for o in out[1:]:
+            assert all(np.array_equal(a, b, equal_nan=True) for a, b in zip(o, out[0])), k
+        P = ctx[0][0].get("P")
+        for dev, _ in ctx:
+            dev.set("P", np.round(P * 1.01, 3))
+    for dev, _ in ctx:
+        dev.close()
