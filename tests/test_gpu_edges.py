@@ -1,9 +1,12 @@
 """Edge cases of the device path against the oracle: the smallest and
 largest component counts the kernels are built for, a single cell without
 connections, and a grid without cells."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
+from opencaeporox_amd import abi
 from opencaeporox_amd import workload as W
 from opencaeporox_amd.fim import BATCHED, PLAIN, IsoTFIM
 from oracle.oracle import state_from_workload
@@ -204,3 +207,35 @@ def test_one_lane_kernel_takes_every_cell_once(nb):
             dev.set("P", np.round(P * 1.01, 3))
     for dev, _ in ctx:
         dev.close()
+
+
+@pytest.mark.parametrize("nb", [1, 64, 30000])
+def test_new_context_on_a_stream_not_ordered_with_the_default_one(nb):
+    """New buffers are zeroed before anything else reaches them: what is uploaded
+    at creation, the first saved time step, the first flash's lists, the wells."""
+    from opencaeporox_amd import wells as WL
+    stream = C.c_void_p()
+    assert abi.load().hipStreamCreateWithFlags(C.byref(stream), 1) == 0        # hipStreamNonBlocking
+    wl = _repeated(6, 1501, nb)
+    wells = [WL.PeacemanWell("P", WL.PROD, WL.BHP, bhp=1.0, target=1.0, cells=[nb // 2], WI=[2.0])]
+    out = []
+    for st in (None, stream):
+        dev = IsoTFIM.from_workload(wl, stream=st)
+        dev.UpdateLastTimeStep()
+        got = {f: dev.get(f) for f in ("P", "NI", "FTYPE_IN", "DSEC_DPRI")}
+        dev.CalFlash(BATCHED)
+        dev.SetWells(wells)
+        dev.CalKrPc()
+        dev.CalRock()
+        dev.AssembleMatBulks(1.0)
+        got["norms"], got["wres"] = dev.CalResWells(1.0, jacobian=True)
+        for f in ("ITERS", "PHASEEXIST", "XIJ", "DSEC_DPRI"):
+            got[f + " after"] = dev.get(f)
+        dev.ResetToLastTimeStep()
+        got.update({f + " reset": dev.get(f) for f in ("P", "NI", "XIJ", "ITERS")})
+        dev.close()
+        out.append(got)
+    for f in out[0]:
+        assert np.array_equal(out[0][f], out[1][f], equal_nan=True), f
+    assert np.any(out[0]["P reset"] > 0) and np.any(out[0]["ITERS after"] > 0)
+    assert abi.load().hipStreamDestroy(stream) == 0
