@@ -224,3 +224,98 @@ def test_solve_after_new_transmissibilities_on_a_callers_stream():
         fresh.close()
     dev.close()
     assert abi.load().hipStreamDestroy(stream) == 0
+
+
+def _cpr_case(Nc, dims, sigma, odd=False):
+    rng = np.random.Generator(np.random.PCG64(17))
+    nx, ny, nz = dims
+    nb = nx * ny * nz
+    k = np.exp(rng.normal(np.log(100.0), sigma, nb))
+    grid = W.cartesian_grid(nx, ny, nz, 6.096, k, k, 0.1 * k, rng.uniform(0.1, 0.3, nb))
+    if odd:
+        grid = _odd_cycle(grid, nx)
+    fl, rock = W.make_fluid(Nc, 103), W.make_rock()
+    z = np.tile(rng.dirichlet(np.ones(Nc)), (nb, 1))
+    st = W.initial_state(fl, rock, grid, 200.0 + rng.normal(0, 5.0, nb), z, rng)
+    return W.Workload("cpr", fl, W.make_sat(), rock, grid, st)
+
+
+def _decoupled_residual(D, J, rhs, u):
+    """||D^-1 (rhs - J u)|| / ||D^-1 rhs|| with the diagonal blocks D."""
+    b = D.shape[1]
+    solve = lambda v: np.linalg.solve(D, v.reshape(-1, b, 1)).ravel()
+    return np.linalg.norm(solve(rhs - J @ u)) / np.linalg.norm(solve(rhs))
+
+
+def test_cpr_on_long_vectors_past_a_restart():
+    """Vectors of more than 1,048,576 entries, no multiple of a tile, over more than the 30 iterations to a
+    restart: the basis kernels of long vectors at every number of basis vectors, checked on the host."""
+    wl = _cpr_case(6, (61, 57, 43), 2.0)
+    dev = IsoTFIM.from_workload(wl)
+    dev.newton_pass(0.01, BATCHED)
+    assert dev.nb * dev.bs > 512 * 256 * 8 and dev.nb * dev.bs % 2048
+    J, rhs = _system(dev)
+    rp, _, val, _ = dev.bsr()
+    u, it, rr = dev.LinearSolve(rtol=1e-11, maxit=200)
+    res = _decoupled_residual(val[rp[:-1]], J, rhs, u)
+    print(f"61x57x43: {it} iterations, decoupled residual {rr:.2e}, on the host {res:.2e}")
+    assert it > 30 and rr < 1e-11
+    # the device stops on its own value of this residual; the host's differs by rounding
+    assert res < 2e-11
+    dev.close()
+
+
+@pytest.mark.parametrize("odd", [False, True])
+@pytest.mark.parametrize("Nc,dims", [(3, (7, 6, 5)), (6, (16, 9, 8))])
+def test_cpr_with_wells_over_colours(Nc, dims, odd):
+    """The wells' rows beside both sweeps, the two-coloured one and the one for any number of colours."""
+    from opencaeporox_amd import wells as WL
+    wl = _cpr_case(Nc, dims, 1.0, odd)
+    wells = WL.corner_and_centre_wells(wl)
+    dev = IsoTFIM.from_workload(wl)
+    dev.SetWells(wells)
+    dev.newton_pass(0.01, BATCHED)
+    _, wres = dev.CalResWells(0.01, jacobian=True)
+    rp, col, val, rhs = dev.bsr()
+    J, f = WL.full_system(rp, col, val, rhs, wells, *dev.well_blocks(), wres, dev.bs)
+    u, it, rr = dev.LinearSolve(rtol=1e-11, maxit=200)
+    true = np.linalg.norm(f - J @ u) / np.linalg.norm(f)
+    ref = spla.spsolve(J.tocsc(), f)
+    err = np.linalg.norm(u - ref) / np.linalg.norm(ref)
+    print(f"{dims} Nc={Nc} odd={odd} with wells: {it} iterations, true {true:.2e}, error {err:.2e}")
+    assert it > 0 and rr < 1e-11
+    # as test_cpr_over_grids_and_colours
+    assert true < 1e-9 and err < 1e-6
+    dev.close()
+
+
+@pytest.mark.parametrize("odd", [False, True])
+def test_cpr_with_ill_conditioned_diagonal_blocks(odd):
+    """The rows of a tenth of the cells multiplied by matrices of condition 1e8: the decoupled system is the
+    same, the diagonal blocks are not.  Both sweeps solve it as before; the inverse of such a block is
+    off by 1e-16 times its condition, of which little reaches the residual (1e-8 of it here)."""
+    dev = IsoTFIM.from_workload(_cpr_case(6, (13, 12, 9), 1.0, odd))
+    dev.newton_pass(0.01, BATCHED)
+    J, rhs = _system(dev)
+    rp, _, val, _ = dev.bsr()
+    b, nb = dev.bs, dev.nb
+    D = val[rp[:-1]]
+    _, it0, _ = dev.LinearSolve(rtol=1e-6, maxit=200)
+    rng = np.random.Generator(np.random.PCG64(3))
+    rhs1, val1 = rhs.reshape(nb, b).copy(), val.copy()
+    for n in rng.choice(nb, nb // 10, replace=False):
+        q, r = (np.linalg.qr(rng.normal(size=(b, b)))[0] for _ in range(2))
+        S = (q * np.logspace(0, -8, b)) @ r
+        rhs1[n] = S @ rhs1[n]
+        val1[rp[n]:rp[n + 1]] = S @ val1[rp[n]:rp[n + 1]]
+    lib = abi.load()
+    ptr = [C.c_void_p() for _ in range(4)]
+    assert lib.ocpx_bsr_device_ptrs(dev.h, *[C.byref(p) for p in ptr]) == 0
+    dev.sync()
+    for p, a in ((ptr[2], val1), (ptr[3], rhs1)):
+        assert lib.hipMemcpy(p, C.c_void_p(a.ctypes.data), C.c_size_t(a.nbytes), C.c_int(1)) == 0
+    u, it, rr = dev.LinearSolve(rtol=1e-6, maxit=200)
+    res = _decoupled_residual(D, J, rhs, u)
+    print(f"odd={odd}: {it0} iterations, {it} with ill-conditioned blocks, residual {rr:.2e}, {res:.2e}")
+    assert 0 < it <= it0 + 1 and rr < 1e-6 and res < 2e-6
+    dev.close()
