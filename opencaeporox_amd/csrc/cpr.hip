@@ -188,11 +188,12 @@ __global__ void __launch_bounds__(256) amg_up(int64_t nq, const int64_t* __restr
     xo[i] = (x[i] + xc[q >> 2]) + OMEGA * dinv[i] * r;
 }
 
-// The part of the V-cycle below about 2,000 rows in one workgroup: every
-// vector in LDS, the matrices read from L2, the coarsest level by its dense
-// inverse.  Launched level by level, those levels took four launches each and
-// a serial triangular solve (27 us), about 150 us of the cycle's 550 at
-// 500,000 rows; this kernel takes 25.
+// The part of the V-cycle from the first level of at most SM_TOP rows on (levels
+// of at most SM_ROWS together) in one workgroup: every vector in LDS, the
+// matrices read from L2, the coarsest level by its dense inverse.  Launched level
+// by level, the levels below 2,000 rows took four launches each and a serial
+// triangular solve (27 us), about 150 us of the cycle's 550 at 500,000 rows; this
+// kernel takes 25.
 constexpr int SM_ROWS = 1536, SM_TOP = 1024, SM_LEVELS = 14, SM_THREADS = 1024;
 struct SmallLevel {
     int n, nc, nq;
@@ -404,6 +405,8 @@ __global__ void __launch_bounds__(64) cpr_resid(const int64_t* __restrict__ rowp
 // colour's are g2 = R2 - Dinv A21 R1 (SECOND), z = g + x1.  Then w = D^{-1} J z =
 // D^{-1} J g + (v - R); the sweep solved the second colour's rows exactly, so w2 =
 // v2, and w1 = R1 + Dinv A12 g2 + v1 - R1 = v1 + Dinv A12 g2 (first colour).
+// That takes Dinv D for the identity, which it is to eps cond(D); a product with
+// D and then Dinv rounds by as much.
 // R holds g afterwards.  One iteration reads the off-diagonal blocks once; the
 // sweep over both colours, the residual before it and the product after it read
 // the matrix three times (500,000 rows, B = 8: 0.47 + 0.36 + 0.36 ms, now 0.41, at

@@ -16,8 +16,8 @@
 //    aggregates of up to four cells); every solve forms the level matrices
 //    on the device (level 0 from the BSR, coarser ones by Galerkin sums over
 //    a precomputed gather list) and applies one V-cycle: one weighted-Jacobi
-//    sweep before and after the coarse correction, a dense LU on the
-//    coarsest level.
+//    sweep before and after the coarse correction, a product with the dense
+//    inverse (formed once per solve) on the coarsest level.
 //  * the second stage: one multicolour block Gauss-Seidel sweep on the
 //    decoupled system (whose diagonal blocks are the identity), colours
 //    from a greedy colouring of the block graph.  With two colours (any

@@ -303,7 +303,7 @@ int sta_alloc(ocpx_ctx* c)
     auto part = [&](auto** p, size_t count) { parts.emplace_back((void**)p, (count * sizeof(**p) + 255) & ~(size_t)255); };
     part(&cnt, 16);
     part(&s.glist, n); part(&s.route, n); part(&s.decided, n); part(&s.defer, n); part(&s.stop, n); part(&s.Ytd, 4 * n);
-    part(&s.evals, n); part(&s.its, 4 * n); part(&s.item, 4 * n); part(&s.di, (size_t)c->NC * n);
+    part(&s.its, 4 * n); part(&s.item, 4 * n); part(&s.di, (size_t)c->NC * n);
     part(&s.nr_cell, cap); part(&s.nr_k, cap); part(&s.nr_flag, cap); part(&s.nr_its, cap); part(&s.nr_evals, cap);
     part(&s.nr_Yt, cap); part(&s.nr_y, (size_t)c->NC * cap); part(&s.rs_Yt, n); part(&s.rs_cnt, 8 * n);
     part(&s.slist, n); part(&s.tlist, n); part(&s.llist, n); part(&s.rs_v, (size_t)5 * c->NC * n); part(&s.rs_nu, n);

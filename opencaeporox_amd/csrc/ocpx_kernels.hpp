@@ -86,7 +86,6 @@ struct StaIO {
     int32_t* decided;           // [nb] not apart: first trial stage 1 found unstable, 4 none
     int32_t* defer;             // [nb] not apart: bit k: trial k queued for its Newton step
     double* Ytd;                // [nb], apart [4][nb]: Yt of the trial(s) stage 1 found unstable
-    int32_t* evals;             // [nb] stage-1 fugacity evaluations
     int32_t* its;               // [4][nb] SSM iterations per trial
     int32_t* item;              // [4][nb] Newton item of a queued trial; apart: else -1 stable, -2 unstable
     double* di;                 // [Nc][nb] phi * z of the feed
